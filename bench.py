@@ -44,9 +44,9 @@ def sparse_kernel_bytes(T, E_raw, nsel, nrows, n_mapped, tuning, px, ev, tdeep=N
 
     px / ev: pixels and level-0 events per row class (plan.row_stats(): empty,
     1..64, 65..128, 129..512, 513..2048, longer).  Row classes and their
-    kernels: empty and 1..64 -> the k_mt_reg timer (the classification pass,
-    which lists the others at 4 B each, and the register kernel); 65..2048 ->
-    the k_mt_lds timer (k_mt_reg2 and the two LDS kernels); longer ->
+    kernels: empty and 1..64 -> the k_mt_reg timer (the row kernel over rows
+    in place); 65..2048 -> the k_mt_lds timer (the row kernels over the lists
+    of the classification pass, 4 B an entry, and the LDS kernel); longer ->
     k_mt_long.  Per row kernel: its rows' events (8 B), compact-to-row map
     (4 B) and row offsets (2 x 8 B) in, the int64 G2 and the 32-bit IP/IF
     of every tau (16 B per tau; pixels whose total passes 2^32 - 1, none
@@ -715,7 +715,7 @@ def run_job(name, steps, warmup, autotune=True, e2e=True):
         lev = np.asarray(levels)
         tdeep = int((lev < info.deep_level).sum())
         abytes = sparse_kernel_bytes(T, int(dlen.sum()), len(dlen), W * H, info.mapped_pixels, shapes, px, ev,
-                                     tdeep if info.deep_stride > 0 else None, info.deep_stride)
+                                     tdeep if "k_mt_deep" in ktimes else None, info.deep_stride)
     kern = {}
     for k, (ms, n) in ktimes.items():
         avg_ms = ms / max(n, 1)

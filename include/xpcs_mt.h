@@ -98,9 +98,9 @@ typedef struct xpcs_mt_info {
     int64_t long_pixels;        /* dense ingests: every pixel (dense-row or
                                    streaming kernels); sparse: pixels whose rows
                                    hold more than 1024 events                 */
-    int32_t deep_level;         /* sparse path: first level of the one-lane-per-pixel
-                                   kernel (levels above it; = level count: none) */
-    int32_t deep_stride;        /* its series row, u32 values per pixel (0: none) */
+    int32_t deep_level;         /* sparse path, rows of at most 64 events: first level
+                                   summed from the dense series (= level count: none) */
+    int32_t deep_stride;        /* values of that series (0: none) */
 } xpcs_mt_info;
 
 /* Library version string. */
@@ -354,11 +354,13 @@ xpcs_status xpcs_mt_set_timing_filter(xpcs_mt_plan* plan, const char* name);
  *   dense_levels     levels per pass of the dense streaming kernel, i.e. the
  *                    depth of its register-resident lag window
  *                    (dpl 4: 3, 4, 5; dpl 8: 2, 3)
- *   deep_frames      sparse rows of at most 128 events hand their levels over
- *                    to a one-lane-per-pixel kernel from the first level with
- *                    at most deep_frames binned frames (16..96; negative: no
- *                    hand-over; 0: 96).  Only for dpl 4 or 8, T <= 128 and at
- *                    most 48 taus from that level on (otherwise no hand-over).
+ *   deep_frames      sparse rows are summed as dense series from the first
+ *                    level with at most deep_frames binned frames (16..96;
+ *                    negative: never; 0: three frames per event of the row's
+ *                    length class).  Only for dpl 4 or 8.  Plans of more than
+ *                    about 64,000 frames hand rows of at most 128 events over
+ *                    to a kernel of their own there (0: 96; T <= 128 and at
+ *                    most 48 taus from that level on, otherwise no hand-over).
  *   sums64           0: integer IP and IF sums are kept on the device as 32-bit
  *                    words plus the high words of the pixels whose total
  *                    passes 2^32 - 1 (the normalisation reads 16 instead of

@@ -298,7 +298,7 @@ extern "C" xpcs_status xpcs_mt_plan_destroy(xpcs_mt_plan* p)
     dfree(p->d_q_chunk_first); dfree(p->d_q_first_group); dfree(p->d_weight); dfree(p->d_c2pix);
     dfree(p->d_sbin_of_c); dfree(p->d_sbin_pix); dfree(p->d_imm_owned); dfree(p->d_sel_off); dfree(p->d_sel_dlen);
     dfree(p->d_sel_frame); dfree(p->d_dark_sum); dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_off);
-    dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_counters);
+    dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_wide_list); dfree(p->d_counters);
     dfree(p->d_scratch); dfree(p->d_G2); dfree(p->d_IP); dfree(p->d_IF); dfree(p->d_pix_total); dfree(p->d_fw);
     dfree(p->d_deep);
     dfree(p->d_part); dfree(p->d_g2s); dfree(p->d_g2); dfree(p->d_se); dfree(p->d_fs); dfree(p->d_series_a); dfree(p->d_series_b); dfree(p->d_bnd);
@@ -923,8 +923,10 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
         }
         if (row_off[j + 1] - row_off[j] <= reg_cap() && tot > 0xFFFFFFFFull) wide = true;
     }
-    xpcs_status st = upload(&p->d_ev, ev, p->stream);
+    xpcs_status st = dalloc(&p->d_ev, ev.size() + kRowSlack);
     if (st) return st;
+    if (!ev.empty())
+        HIP_TRY(hipMemcpyAsync(p->d_ev, ev.data(), ev.size() * sizeof(uint64_t), hipMemcpyHostToDevice, p->stream));
     p->ev_cap = (int64_t)ev.size();
     HIP_TRY(hipMemcpyAsync(p->d_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice, p->stream));
     p->events = off[(size_t)h.P];
@@ -965,7 +967,12 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
         xpcs_status st = dalloc(&p->d_scratch, (size_t)p->long_blocks * h.F);
         if (st) return st;
     }
-    if (p->mode == 1 || p->mode == 3) {
+    if ((p->mode == 1 || p->mode == 3) && rows_supported(p)) {
+        if (!p->d_wide_list) {
+            xpcs_status st = dalloc(&p->d_wide_list, (size_t)h.P);
+            if (st) return st;
+        }
+    } else if (p->mode == 1 || p->mode == 3) {
         rank_lds_setup(p);
         int stride = 0;
         if (deep_level(p, &stride) < (int)h.levels.size()) {
@@ -978,8 +985,8 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
         }
     }
     if (p->mode == 1) {
-        if (p->raw_events > p->ev_cap) {
-            xpcs_status st = dalloc(&p->d_ev, (size_t)p->raw_events);
+        if (!p->d_ev || p->raw_events > p->ev_cap) {
+            xpcs_status st = dalloc(&p->d_ev, (size_t)p->raw_events + kRowSlack);
             if (!st) st = dalloc(&p->d_b1, (size_t)p->raw_events);
             if (st) return st;
             p->ev_cap = p->raw_events;

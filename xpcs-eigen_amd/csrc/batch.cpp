@@ -95,7 +95,7 @@ extern "C" xpcs_status xpcs_mt_get_tuning(xpcs_mt_plan* p, xpcs_mt_tuning* t)
     t->reg_blocks = reg_blocks(p);
     t->lds_blocks = lds_blocks(p);
     t->dense_levels = (p->h.dpl == 4 || p->h.dpl == 8) ? dense_levels(p) : 0;
-    t->deep_frames = p->tune.deep_frames < 0 ? -1 : (p->tune.deep_frames > 0 ? p->tune.deep_frames : 96);
+    t->deep_frames = p->tune.deep_frames < 0 ? -1 : (p->tune.deep_frames > 0 ? p->tune.deep_frames : rows_supported(p) ? 0 : 96);
     t->sums64 = p->tune.sums64;
     return XPCS_OK;
 }

@@ -18,6 +18,8 @@ constexpr int kWave = 64;
 constexpr int kSparseCap = 1024;
 // Largest schedule supported by the per-wave LDS accumulators.
 constexpr int kMaxTaus = 256;
+// Events past the end of the event buffer that the row kernels may read (and discard).
+constexpr int kRowSlack = 1024;
 
 // One schedule entry as the kernels need it.
 struct TauParam {
@@ -205,8 +207,10 @@ struct xpcs_mt_plan {
     // long pixels
     int32_t* d_long_list = nullptr;      // [P]
     int32_t* d_mid_list = nullptr;       // [P] rows of 65..CAP events
+    int32_t* d_wide_list = nullptr;      // [P] rows of at most 1024 events whose total passes 65535
     uint32_t* d_counters = nullptr;      // [0] rows over 1024 events, [1] error flags, [2] rows of 65..128,
-                                         // [3] dense exact-redo pixels, [4] rows of 129..512, [5] 513..1024
+                                         // [3] dense exact-redo pixels, [4] rows of 129..512, [5] 513..1024,
+                                         // [6] rows in d_wide_list
     uint32_t* d_deep = nullptr;          // [P][deep stride] level series handed to the one-lane-per-pixel kernel
     size_t deep_cap = 0;
     uint64_t* d_scratch = nullptr;
@@ -265,6 +269,11 @@ constexpr int64_t kSideFuseDoubles = 4096;   // LDS frame-sum table of the fused
 bool side_fused(const xpcs_mt_plan* p);
 EvFormat ev_format(const xpcs_mt_plan* p);
 void launch_mt_sparse(xpcs_mt_plan* p, hipStream_t s);
+// k_rows.hip: rows of at most 1024 events, a group of lanes per row; rows
+// whose total passes 65535 are left in d_wide_list
+bool rows_supported(const xpcs_mt_plan* p);
+int rows_series_level(const xpcs_mt_plan* p, int N);
+void launch_mt_rows(xpcs_mt_plan* p, hipStream_t s);
 // first level of the one-lane-per-pixel kernel of the sparse path (the level
 // count: none) and its series row length in u32 (0: none)
 int deep_level(const xpcs_mt_plan* p, int* stride);

@@ -9,6 +9,10 @@
 //   IF = sum_{tau'<=t<lf_L} x_L[t] = S0(2^L lf_L) - S0(2^L tau'),
 // where S0(b) is the sum of the level-0 counts of frames < b.
 //
+// Rows of counts at 4 or 8 delays per level go through k_mt_rows (k_rows.hip)
+// unless the row total passes 65535 or the plan's frames its 16-bit keys; the
+// kernels here take the rest, and the FP64 frame-weighted values.
+//
 // k_mt_reg / k_mt_reg2: one wavefront per row of at most 64 / 128 events held
 // in registers (one / two per lane).  The row is sorted (odd-even passes, a
 // bitonic network when still unsorted), duplicates merged, IP/IF taken from
@@ -1786,11 +1790,32 @@ static void launch_rows(xpcs_mt_plan* p, hipStream_t s, const char* t_reg, const
     // register rows (32-bit level values): T <= kRegMaxTaus, and no row of at
     // most kMidSmall events totals 2^32 or more (pixel-major rows of u32 counts)
     const bool regs = h.T <= kRegMaxTaus && !(p->mode == 3 && p->wide_rows);
+    const bool rows = sizeof(V) == 4 && rows_supported(p);
     timer_begin(p, s, "k_mt_classify");
     if (h.P > 0)
         k_mt_classify<<<(unsigned)((h.P + 256 * kClassifyPer - 1) / (256 * kClassifyPer)), 256, 0, s>>>(
-            p->d_off, p->d_rowmap, h.P, regs, p->d_mid_list, p->d_long_list, p->d_counters);
+            p->d_off, p->d_rowmap, h.P, regs || rows, p->d_mid_list, p->d_long_list, p->d_counters);
     timer_end(p, s);
+    if (rows) {
+        launch_mt_rows(p, s);
+        const int nl = (int)h.levels.size();
+        const int64_t hwords = (int64_t)h.P * h.T;
+        timer_begin(p, s, t_lds);
+        k_mt_sparse<kSparseCapMid, kSparseMidWaves, V><<<256, kWave * kSparseMidWaves, 0, s>>>(
+            p->d_ev, p->d_off, p->d_wide_list, 1, p->d_counters + 6, p->d_taus, h.T, p->d_levels, nl, h.F, p->d_G2,
+            p->d_IP, p->d_IF, p->d_pix_total, p->d_rowmap, fw, nl, p->d_deep, 0, p->ipif32, hwords);
+        k_mt_sparse<kSparseCapLong, kSparseLongWaves, V><<<std::max(1, lds_blocks(p) / 4), kWave * kSparseLongWaves, 0, s>>>(
+            p->d_ev, p->d_off, p->d_long_list + (h.P - 1), -1, p->d_counters, p->d_taus, h.T, p->d_levels, nl, h.F,
+            p->d_G2, p->d_IP, p->d_IF, p->d_pix_total, p->d_rowmap, fw, nl, p->d_deep, 0, p->ipif32, hwords);
+        timer_end(p, s);
+        timer_begin(p, s, t_long);
+        k_mt_long<uint64_t><<<p->long_blocks, kLongBlock, 0, s>>>(
+            p->d_ev, p->d_off, p->d_rows, h.P, h.T, p->d_levels, nl, h.F, p->d_long_list + (h.P - 1), -1,
+            (int64_t)kSparseCapLong, p->d_counters, 0, nullptr, p->d_scratch, p->d_G2, p->d_IP, p->d_IF,
+            p->d_pix_total, p->d_rowmap, p->ipif32);
+        timer_end(p, s);
+        return;
+    }
     timer_begin(p, s, t_reg);
     // the deep levels' hand-over (counts only)
     const int nlev = (int)h.levels.size();
@@ -1865,7 +1890,8 @@ static void launch_rows(xpcs_mt_plan* p, hipStream_t s, const char* t_reg, const
     }
 }
 
-// First level of the one-lane-per-pixel kernel: the first level L >= 1 with
+// First level summed from the dense series: in the row kernels, or in the
+// one-lane-per-pixel kernel, there the first level L >= 1 with
 // at most deep_frames binned frames (tuning; 0: kDeepMaxFrames, negative:
 // none), for counts (not the FP64 frame-sum mode), dpl 4 or 8 (the kernel's
 // instantiations), T <= kRegMaxTaus (the register kernels run) and at most
@@ -1875,6 +1901,12 @@ int deep_level(const xpcs_mt_plan* p, int* stride)
     const HostTables& h = p->h;
     const int nlev = (int)h.levels.size();
     *stride = 0;
+    if (rows_supported(p)) {
+        // the row kernels' series form (rows of at most 64 events)
+        const int L = rows_series_level(p, kWave);
+        *stride = L < nlev ? h.levels[(size_t)L].lf : 0;
+        return L;
+    }
     const int lim = p->tune.deep_frames < 0 ? 0 : (p->tune.deep_frames > 0 ? p->tune.deep_frames : kDeepMaxFrames);
     if (lim == 0 || p->fsnorm || (h.dpl != 4 && h.dpl != 8) || h.T > kRegMaxTaus) return nlev;
     for (int L = 1; L < nlev; L++) {
