@@ -192,6 +192,9 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
             words_ok = r == rank[(size_t)f];
         }
         TRY(upload(&p->d_tau_bnd, tj, s));
+        std::vector<int32_t> cap(b);
+        cap.push_back(INT32_MAX);
+        TRY(upload(&p->d_cap, cap, s));
         TRY(upload(&p->d_frame_rank, rank, s));
         if (words_ok && nw > 0) {
             TRY(upload(&p->d_rank_words, words, s));
@@ -298,10 +301,10 @@ extern "C" xpcs_status xpcs_mt_plan_destroy(xpcs_mt_plan* p)
     dfree(p->d_q_chunk_first); dfree(p->d_q_first_group); dfree(p->d_weight); dfree(p->d_c2pix);
     dfree(p->d_sbin_of_c); dfree(p->d_sbin_pix); dfree(p->d_imm_owned); dfree(p->d_sel_off); dfree(p->d_sel_dlen);
     dfree(p->d_sel_frame); dfree(p->d_dark_sum); dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_off);
-    dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_wide_list); dfree(p->d_counters);
+    dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_wide_list); dfree(p->d_wave_flags); dfree(p->d_counters);
     dfree(p->d_scratch); dfree(p->d_G2); dfree(p->d_IP); dfree(p->d_IF); dfree(p->d_pix_total); dfree(p->d_fw);
     dfree(p->d_deep);
-    dfree(p->d_part); dfree(p->d_g2s); dfree(p->d_g2); dfree(p->d_se); dfree(p->d_fs); dfree(p->d_series_a); dfree(p->d_series_b); dfree(p->d_bnd);
+    dfree(p->d_part); dfree(p->d_g2s); dfree(p->d_g2); dfree(p->d_se); dfree(p->d_fs); dfree(p->d_series_a); dfree(p->d_series_b); dfree(p->d_bnd); dfree(p->d_cap);
     for (auto& t : p->pending) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     for (auto e : p->event_pool) (void)hipEventDestroy(e);
     twotime_release(p);
@@ -557,7 +560,19 @@ void dense_tiling(xpcs_mt_plan* p, const std::vector<int64_t>& so, const uint8_t
     p->side_vec = npd % 8 == 0;
     for (int64_t o : so)
         if (((uintptr_t)base + (uintptr_t)o) % 16 != 0) p->side_vec = false;
-    if (h.avg != 1 || so.empty() || npd % 8 != 0) return;
+    p->even_off0 = -1;
+    p->even_step = 0;
+    if (h.avg != 1 || so.empty()) return;
+    {
+        const int64_t d = so.size() > 1 ? so[1] - so[0] : 0;
+        bool even = d >= 0 && ((uintptr_t)base + (uintptr_t)so[0]) % 2 == 0 && d % 2 == 0;
+        for (size_t k = 0; k < so.size() && even; k++) even = so[k] == so[0] + (int64_t)k * d;
+        if (even) {
+            p->even_off0 = so[0];
+            p->even_step = d;
+        }
+    }
+    if (npd % 8 != 0) return;
     const int64_t step = so.size() > 1 ? so[1] - so[0] : 16;
     if (step <= 0 || step % 16 != 0 || ((uintptr_t)base + (uintptr_t)so[0]) % 16 != 0) return;
     for (size_t k = 0; k < so.size(); k++)
@@ -1011,6 +1026,11 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
             p->bsum_cap = nbs;
         }
     } else if (dense_stream) {
+        if (!p->d_wave_flags) {
+            // one flag per wave of the dense kernels' grids (whole workgroups of 256)
+            xpcs_status st = dalloc(&p->d_wave_flags, ((size_t)h.W * h.H + 255) / 256 * 4);
+            if (st) return st;
+        }
         const size_t need = dense_series_elems(p);
         if (need > p->series_cap) {
             xpcs_status st = dalloc(&p->d_series_a, need);

@@ -146,6 +146,10 @@ struct xpcs_mt_plan {
     uint32_t* d_mapped = nullptr;        // bit per detector pixel: dqmap, sqmap >= 1
     int64_t tile_off0 = -1;
     int64_t tile_step = 0;
+    // the same spacing at any alignment (frames of one raw frame each); -1 otherwise
+    int64_t even_off0 = -1;
+    int64_t even_step = 0;
+    uint32_t* d_wave_flags = nullptr;    // per 64 detector pixels: left to the FP64 dense kernel
     bool side_vec = false;   // every selected dense frame 16-byte aligned, pixels % 8 == 0
     int64_t nsel = 0;                    // selected raw frames
     int64_t* d_sel_off = nullptr;        // payload byte offset per selected raw frame
@@ -193,6 +197,7 @@ struct xpcs_mt_plan {
     size_t series_cap = 0;
     int4* d_bnd = nullptr;               // (frame boundary, op, tau slot, 0), sorted
     int32_t nbnd = 0;
+    int32_t* d_cap = nullptr;            // the distinct boundaries B_j and an entry beyond every frame
     // distinct prefix-sum boundaries B_j of the sparse row kernels (sorted)
     uint16_t* d_frame_rank = nullptr;    // [F] number of B_j <= frame
     int4* d_tau_bnd = nullptr;           // [T] (j of IP, j of the IF head, j of the level end, 0)

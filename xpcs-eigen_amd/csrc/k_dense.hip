@@ -165,10 +165,12 @@ k_mt_dense_f64(const uint8_t* __restrict__ imm, const int64_t* __restrict__ sel_
                int64_t* __restrict__ IF, uint64_t* __restrict__ pix_total,
                std::conditional_t<FP, double, uint32_t>* __restrict__ series_out, uint32_t lf_out,
                uint32_t* __restrict__ redo_count, int32_t* __restrict__ redo_list, const double* __restrict__ fw,
-               bool w32)
+               bool w32, const uint32_t* __restrict__ only)
 {
     using ST = std::conditional_t<FP, double, uint32_t>;   // series element
     constexpr bool RAW = MODE != kSeries;
+    // only: a flag per 64 pixels; waves without it have nothing to do
+    if (RAW && only && only[(blockIdx.x * blockDim.x + threadIdx.x) >> 6] == 0u) return;
     // values of a group: integers from the raw frames, or the input series
     using XT = std::conditional_t<FP && !RAW, double, uint32_t>;
     constexpr bool TILES = MODE == kRawTiles;
@@ -417,6 +419,410 @@ k_mt_dense_f64(const uint8_t* __restrict__ imm, const int64_t* __restrict__ sel_
                 if (d >= dlo && rel >= 0 && rel < lp.count)
                     G2[rowT + lp.first + rel] =
                         FP ? (int64_t)__double_as_longlong(s.acc[l][d - 1]) : (int64_t)s.acc[l][d - 1];
+            }
+        }
+    }
+}
+
+// ---- raw pass over counts: two-element dot products --------------------------
+// The same streaming pass (thread per pixel, 16-frame groups, K levels) with
+// the values of two consecutive frames in one register: a lag sum takes one
+// two-element integer dot product per two frames (even lags against earlier
+// words, odd lags against words one frame off) instead of two FP64
+// multiply-adds, the pair sums and the running total are dot products with
+// (1, 1), and dark subtraction and threshold work on both halves at once.
+//
+// Lag sums run in 32 bits and are added to the FP64 totals (flush) before they
+// could overflow: a chunk between flushes holds at most kDotChunk counts per
+// pixel, the 68 frames before it (five groups, the deepest lag) at most five
+// times that, and kDotChunk (kDotChunk + 5 kDotChunk) < 2^32; kDotChunk also
+// keeps every value of a group's levels in 16 bits.  A wave that meets a
+// 16-frame group beyond kDotChunk in any pixel flags its 64 pixels and stops;
+// the FP64 kernel then takes exactly those.
+//
+// The FP64 form was bound by vector issue (20 instructions per frame and
+// wave, two waves per SIMD); measured on the 512 x 512 x 20,000-frame job
+// (dpl 4, two darks): 3.45 -> 2.58 ms (11 GB of HBM traffic, 4.3 TB/s: memory
+// now bounds it), on 333 x 251 x 3001 frames (dpl 8) 1.04 -> 0.36 ms.
+constexpr uint32_t kDotChunk = 26000u;
+using u16x2 = __attribute__((ext_vector_type(2))) unsigned short;
+using i16x2 = __attribute__((ext_vector_type(2))) short;
+
+__device__ __forceinline__ uint32_t dot2_u16(uint32_t a, uint32_t b, uint32_t c)
+{
+    return __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b), c, false);
+}
+
+template <int DPL, int K>
+struct DState {
+    uint32_t win[K][DPL];       // win[l][j]: word j + 1 back at level l
+    uint32_t sh[K][DPL];        // the same one frame earlier: (last of word j + 2 back, first of word j + 1 back)
+    uint32_t acc[K][2 * DPL];   // lag sums since the last flush
+};
+
+// Lags of the first K levels, and the slot of lag d at level l among them.
+template <int DPL, int K>
+constexpr int dot_lags() { return 2 * DPL + (K - 1) * DPL; }
+template <int DPL>
+constexpr int dot_slot(int l, int d) { return l * DPL + d - 1; }
+
+// Lag sums of the NW words of level l.
+template <int DPL, int K, int l, int NW>
+__device__ __forceinline__ void dot_level(DState<DPL, K>& s, const uint32_t (&cur)[NW])
+{
+    constexpr int lo = lag_lo<DPL, true, l>();
+    uint32_t sc[NW];
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+        const uint32_t prev = i > 0 ? cur[i > 0 ? i - 1 : 0] : s.win[l][0];
+        sc[i] = __builtin_amdgcn_alignbit(cur[i], prev, 16);
+#pragma unroll
+        for (int lag = lo; lag <= 2 * DPL; lag++) {
+            const int m = lag / 2;
+            uint32_t w;
+            if (lag & 1) w = m <= i ? sc[m <= i ? i - m : 0] : s.sh[l][m <= i ? 0 : m - i - 1];
+            else w = m <= i ? cur[m <= i ? i - m : 0] : s.win[l][m <= i ? 0 : m - i - 1];
+            s.acc[l][lag - 1] = dot2_u16(cur[i], w, s.acc[l][lag - 1]);
+        }
+    }
+    uint32_t nw[DPL], ns[DPL];
+#pragma unroll
+    for (int j = 0; j < DPL; j++) {
+        nw[j] = j < NW ? cur[j < NW ? NW - 1 - j : 0] : s.win[l][j < NW ? 0 : j - NW];
+        ns[j] = j < NW ? sc[j < NW ? NW - 1 - j : 0] : s.sh[l][j < NW ? 0 : j - NW];
+    }
+#pragma unroll
+    for (int j = 0; j < DPL; j++) {
+        s.win[l][j] = nw[j];
+        s.sh[l][j] = ns[j];
+    }
+}
+
+// The lag sums into the lane's 64-bit totals, tot[slot][lane].
+template <int DPL, int K>
+__device__ __forceinline__ void dot_flush(DState<DPL, K>& s, unsigned long long* tot)
+{
+#pragma unroll
+    for (int l = 0; l < K; l++)
+#pragma unroll
+        for (int d = (l == 0 ? 1 : DPL + 1); d <= 2 * DPL; d++) {
+            atomicAdd(tot + dot_slot<DPL>(l, d) * 64, (unsigned long long)s.acc[l][d - 1]);
+            s.acc[l][d - 1] = 0u;
+        }
+}
+
+__device__ __forceinline__ u16x2 as_pair(uint32_t w) { return __builtin_bit_cast(u16x2, w); }
+__device__ __forceinline__ uint32_t as_word(u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+
+// The next level's word from two words of a level: (a.lo + a.hi, b.lo + b.hi),
+// saturated.  (Dot products with (1, 1) would need wait states before every
+// use.)
+__device__ __forceinline__ uint32_t pair_up(uint32_t a, uint32_t b)
+{
+    const uint32_t lo = __builtin_amdgcn_perm(b, a, 0x05040100u), hi = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    return as_word(__builtin_elementwise_add_sat(as_pair(lo), as_pair(hi)));
+}
+
+struct DotArgs {
+    const uint8_t* src;           // payload of frame t at src + t * step
+    int64_t step;
+    const int32_t* pix2c;
+    uint32_t npix, n_in;
+    const int64_t* dark_sum;
+    const int64_t* thr;
+    int32_t nscale;
+    const LevelParam* levels;
+    int32_t nlev_pass;
+    const int32_t* cap;           // distinct frame boundaries, sorted, and an entry beyond every frame
+    int32_t ncap, T;
+    const int4* tau_bnd;          // per tau: boundary of IP, of the IF head, of the level's end
+    uint32_t* cap_sums;           // [boundary][npix] sums below the boundary
+    int64_t* G2;
+    int64_t* IP;
+    int64_t* IF;
+    uint64_t* pix_total;
+    uint32_t* series_out;
+    uint32_t lf_out;
+    uint32_t* redo_count;
+    int32_t* redo_list;
+    uint32_t* wave_flags;         // per 64 pixels: left to the FP64 kernel
+    bool w32;
+};
+
+struct __attribute__((packed, aligned(2))) Raw8 {
+    uint32_t w[4];
+};
+
+// DARK: n-scaled values y = n raw - sum(dark), kept iff y > max(threshold, 0):
+// with m = floor((max(threshold, 0) + sum(dark)) / n) and t = max(raw - m, 0)
+// that is t > 0 and y = n t + (n m - sum(dark)).  t is limited so that y fits
+// 16 bits; a limited value alone passes kDotChunk.
+//
+// W neighbouring waves to a workgroup and two waves per SIMD: more waves in
+// flight scatter the frame reads (512 x 512 x 20,000 frames, dpl 4: 2.58 ms
+// with 8 waves a workgroup, 2.65 with 4, 2.9 with 1; 3.2 and 3.6 ms at three
+// and four waves per SIMD).  Four tiles in flight: 2.58 against 2.66 ms with
+// three.
+template <int DPL, int K, bool DARK, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_mt_dense_dot(const DotArgs a)
+{
+    constexpr int kDepth = 4;   // 16-frame tiles in flight
+    __shared__ u32x4 s_tile_[W][2 * 64];
+    __shared__ unsigned long long s_tot[W][dot_lags<DPL, K>()][64];
+    const uint32_t lane = threadIdx.x & 63u;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    u32x4* s_tile = s_tile_[w];
+    // consecutive workgroups go to the eight XCDs in turn: each takes a
+    // contiguous eighth of the detector
+    const uint32_t blk = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const uint32_t gid = blk * (64u * W) + threadIdx.x;
+    unsigned long long* tot = &s_tot[w][0][lane];
+    const uint32_t n_in = a.n_in;
+    const int32_t c = gid < a.npix ? a.pix2c[gid] : -1;
+    const bool active = c >= 0;
+    if (lane == 0 && gid < a.npix) a.wave_flags[gid >> 6] = 0u;
+    if (__ballot(active) == 0ull) return;
+    uint32_t rm = 0u, c0 = 0u, tlim = 0u, nsc = 0u;   // in both halves
+    if constexpr (DARK) {
+        const int64_t n = a.nscale;
+        const int64_t ds = active ? a.dark_sum[c] : 0;
+        const int64_t th = active ? a.thr[c] : 0;
+        const int64_t m = min(((th < 0 ? 0 : th) + ds) / n, (int64_t)65535);
+        const int64_t k0 = n * m - ds;
+        const int64_t tl = min((int64_t)32767, (65535 - (k0 > 0 ? k0 : 0)) / n);
+        rm = (uint32_t)m * 0x00010001u;
+        c0 = ((uint32_t)k0 & 0xFFFFu) * 0x00010001u;
+        tlim = (uint32_t)(tl < 0 ? 0 : tl) * 0x00010001u;
+        nsc = ((uint32_t)n & 0xFFFFu) * 0x00010001u;
+    }
+    DState<DPL, K> s;
+#pragma unroll
+    for (int l = 0; l < K; l++) {
+#pragma unroll
+        for (int j = 0; j < DPL; j++) s.win[l][j] = s.sh[l][j] = 0u;
+#pragma unroll
+        for (int j = 0; j < 2 * DPL; j++) {
+            s.acc[l][j] = 0u;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < dot_lags<DPL, K>(); j++) tot[j * 64] = 0ull;
+    const int64_t rowT = (int64_t)(active ? c : 0) * a.T;
+    uint32_t S = 0u, S0 = 0u;      // running total, total at the last flush
+    // Boundaries, two ahead in scalar registers.  Their sums leave frame-major,
+    // a full line per wave: written to the pixels' rows as they came (4 bytes
+    // per pixel, each line revisited ~100 times over the job) they made 18 M
+    // partial HBM writes on the 512 x 512 x 20,000-frame job.
+    using Cap = const __attribute__((address_space(4))) int32_t*;
+    const Cap cap = (Cap)(uintptr_t)a.cap;
+    auto boundary = [&](int i) { return cap[__builtin_amdgcn_readfirstlane(min(i, a.ncap))]; };
+    int bi = 0, cur = boundary(0), nxt = boundary(1);
+    auto capture = [&](uint32_t part) {
+        if (active) a.cap_sums[(int64_t)bi * a.npix + gid] = part;
+        cur = nxt;
+        bi++;
+        nxt = boundary(bi + 1);
+    };
+    while (cur == 0) capture(0u);   // a boundary at frame 0 covers no frames
+
+    // one group; `over` once a pixel of the wave has passed kDotChunk (what the
+    // group then adds is not used)
+    bool over = false;
+    auto group = [&](const uint32_t (&raw)[8], uint32_t t0, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
+        uint32_t x0[8], x1[4], x2[2], x3[1];   // words of levels 0 .. 3
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            uint32_t x = raw[i];
+            if constexpr (DARK) {
+                u16x2 t = __builtin_elementwise_sub_sat(as_pair(x), as_pair(rm));
+                t = __builtin_elementwise_min(t, as_pair(tlim));
+                // all ones where t > 0 (t is below 2^15)
+                const i16x2 kept = (i16x2{0, 0} - __builtin_bit_cast(i16x2, t)) >> 15;
+                const uint32_t add = as_word(__builtin_bit_cast(u16x2, kept)) & c0;
+                x = as_word(t * as_pair(nsc) + as_pair(add));
+            }
+            if constexpr (TAIL) {
+                const uint32_t t = t0 + 2u * (uint32_t)i;
+                x = t + 1 < n_in ? x : t < n_in ? x & 0xFFFFu : 0u;
+            }
+            x0[i] = x;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) x1[i] = pair_up(x0[2 * i], x0[2 * i + 1]);
+#pragma unroll
+        for (int i = 0; i < 2; i++) x2[i] = pair_up(x1[2 * i], x1[2 * i + 1]);
+        x3[0] = pair_up(x2[0], x2[1]);
+        // the group's sum (saturated halves pass kDotChunk)
+        const uint32_t gs = (x3[0] & 0xFFFFu) + (x3[0] >> 16);
+        if constexpr (TAIL) {
+            // values past the end of their level do not exist in its series
+            auto cut = [&](uint32_t* w, int nw, int l) {
+                for (int i = 0; i < nw; i++) {
+                    const uint32_t k = (t0 >> l) + 2u * (uint32_t)i, lim = n_in >> l;
+                    w[i] = k + 1 < lim ? w[i] : k < lim ? w[i] & 0xFFFFu : 0u;
+                }
+            };
+            cut(x1, 4, 1);
+            x2[0] = pair_up(x1[0], x1[1]);
+            x2[1] = pair_up(x1[2], x1[3]);
+            cut(x2, 2, 2);
+            x3[0] = pair_up(x2[0], x2[1]);
+            cut(x3, 1, 3);
+        }
+        if (__ballot(active && S + gs - S0 > kDotChunk) != 0ull) {
+            over = over || __ballot(active && gs > kDotChunk) != 0ull;
+            dot_flush<DPL, K>(s, tot);
+            S0 = S;
+        }
+        // boundary captures (wave-uniform), then the running total
+        while (cur <= (int)(t0 + kGroup)) {
+            const int n = cur - (int)t0;
+            uint32_t part = S;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t ones = n > 2 * i + 1 ? 0x00010001u : n > 2 * i ? 1u : 0u;
+                part = dot2_u16(x0[i], ones, part);
+            }
+            capture(part);
+        }
+        S += gs;
+        dot_level<DPL, K, 0, 8>(s, x0);
+        if constexpr (K > 1) dot_level<DPL, K, 1, 4>(s, x1);
+        if constexpr (K > 2) dot_level<DPL, K, 2, 2>(s, x2);
+        if constexpr (K > 3) dot_level<DPL, K, 3, 1>(s, x3);
+        if (a.lf_out && active) {
+            // level K's values: the sum of 16 frames, or halves of words
+            const uint32_t kb = t0 >> K;
+            uint32_t* o = a.series_out + (int64_t)kb * a.npix + gid;
+#pragma unroll
+            for (int i = 0; i < (16 >> K); i++) {
+                uint32_t v;
+                if constexpr (K == 4) {
+                    v = TAIL ? (kb < a.lf_out ? gs : 0u) : gs;
+                } else {
+                    const uint32_t word = K == 3 ? x3[0] : x2[i >> 1];
+                    v = (i & 1) ? word >> 16 : word & 0xFFFFu;
+                }
+                if (!TAIL || kb + (uint32_t)i < a.lf_out) o[(int64_t)i * a.npix] = v;
+            }
+        }
+    };
+
+    // lane = 8 f + j loads frames t0 + 2 f and t0 + 2 f + 1, pixels 8 j .. 8 j + 7
+    // of the wave; in LDS the tile is [8 frame pairs][64 pixels]
+    uint32_t px = (gid - lane) + 8u * (lane & 7u);
+    const uint32_t back = px + 8u > a.npix ? px + 8u - a.npix : 0u;   // 1..7 for the last pixels' lane
+    px -= back;
+    const bool partial = __builtin_amdgcn_readfirstlane((int)((gid - lane) + 64u > a.npix)) != 0;
+    const uint8_t* src = a.src + 2 * (int64_t)px;
+    auto issue = [&](Raw8 (&r)[2], uint32_t t0) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t t = min(t0 + 2u * (lane >> 3) + (uint32_t)i, n_in - 1);
+            const uint8_t* q = src + (int64_t)t * a.step;
+            r[i] = *reinterpret_cast<const Raw8*>(q);
+        }
+    };
+    auto stage = [&](Raw8 (&r)[2], uint32_t (&x)[8]) {
+        if (partial) {
+            // the detector's last pixels, read from its last 8: move them down
+            // (lanes past the detector keep what they read)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if (back & 1u) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        r[i].w[k] = (r[i].w[k] >> 16) | (k < 3 ? r[i].w[k < 3 ? k + 1 : 3] << 16 : 0u);
+                }
+                if (back & 2u) {
+                    r[i].w[0] = r[i].w[1];
+                    r[i].w[1] = r[i].w[2];
+                    r[i].w[2] = r[i].w[3];
+                }
+                if (back & 4u) {
+                    r[i].w[0] = r[i].w[2];
+                    r[i].w[1] = r[i].w[3];
+                }
+            }
+        }
+        uint32_t q[8];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            q[2 * k] = __builtin_amdgcn_perm(r[1].w[k], r[0].w[k], 0x05040100u);
+            q[2 * k + 1] = __builtin_amdgcn_perm(r[1].w[k], r[0].w[k], 0x07060302u);
+        }
+        s_tile[2 * lane] = u32x4{q[0], q[1], q[2], q[3]};
+        s_tile[2 * lane + 1] = u32x4{q[4], q[5], q[6], q[7]};
+        wave_sync();
+        const uint32_t* t32 = reinterpret_cast<const uint32_t*>(&s_tile[0]);
+#pragma unroll
+        for (int f = 0; f < 8; f++) x[f] = t32[f * 64 + lane];
+        wave_sync();
+    };
+    const uint32_t nfull = n_in / kGroup * kGroup;
+    Raw8 ring[kDepth][2];
+#pragma unroll
+    for (int d = 0; d < kDepth; d++) issue(ring[d], (uint32_t)(d * kGroup));
+    // whole rounds of the ring without a test per tile: a tile skipped on some
+    // path would make every wait drain the loads in flight
+    uint32_t g0 = 0;
+    for (; g0 + kDepth * kGroup <= nfull; g0 += kDepth * kGroup) {
+        if (over) break;
+#pragma unroll
+        for (int d = 0; d < kDepth; d++) {
+            const uint32_t t0 = g0 + (uint32_t)(d * kGroup);
+            uint32_t x[8];
+            stage(ring[d], x);
+            issue(ring[d], t0 + kDepth * kGroup);
+            group(x, t0, std::false_type{});
+        }
+    }
+    for (; g0 < nfull && !over; g0 += kGroup) {
+        uint32_t x[8];
+        stage(ring[0], x);
+#pragma unroll
+        for (int d = 0; d + 1 < kDepth; d++) {
+            ring[d][0] = ring[d + 1][0];
+            ring[d][1] = ring[d + 1][1];
+        }
+        group(x, g0, std::false_type{});
+    }
+    if (!over && nfull < n_in) {
+        Raw8 r[2];
+        issue(r, nfull);
+        uint32_t x[8];
+        stage(r, x);
+        group(x, nfull, std::true_type{});
+    }
+    if (over) {
+        if (lane == 0) a.wave_flags[gid >> 6] = 1u;
+        return;
+    }
+    dot_flush<DPL, K>(s, tot);
+    if (!active) return;
+    a.pix_total[c] = S;
+    // IP = S(B_ip), IF = S(B_end) - S(B_head)
+#pragma unroll 4
+    for (int t = 0; t < a.T; t++) {
+        const int4 b = a.tau_bnd[t];
+        const uint32_t ip = a.cap_sums[(int64_t)b.x * a.npix + gid];
+        const uint32_t head = a.cap_sums[(int64_t)b.y * a.npix + gid], end = a.cap_sums[(int64_t)b.z * a.npix + gid];
+        put_sum(a.IP, rowT + t, (int64_t)ip, a.w32);
+        put_sum(a.IF, rowT + t, (int64_t)end - (int64_t)head, a.w32);
+    }
+    if (S > kExactF64Total) a.redo_list[atomicAdd(a.redo_count, 1u)] = (int32_t)gid;
+#pragma unroll
+    for (int l = 0; l < K; l++) {
+        if (l < a.nlev_pass) {
+            const LevelParam lp = a.levels[l];
+            const int dlo = l == 0 ? 1 : DPL + 1;
+#pragma unroll
+            for (int d = 1; d <= 2 * DPL; d++) {
+                const int rel = d - lp.lo;
+                if (d >= dlo && rel >= 0 && rel < lp.count)
+                    a.G2[rowT + lp.first + rel] = (int64_t)tot[dot_slot<DPL>(l, d) * 64];
             }
         }
     }
@@ -689,13 +1095,64 @@ int dense_levels(const xpcs_mt_plan* p)
     return p->h.dpl == 4 ? dense_levels_per_pass<4>() : dense_levels_per_pass<8>();
 }
 
+// The dot-product raw pass: counts, one raw frame per output frame, evenly
+// spaced frames of any 2-byte alignment, value scales of 16 bits.
+static bool dense_dot_ok(const xpcs_mt_plan* p)
+{
+    return !p->fsnorm && p->even_off0 >= 0 && p->h.avg == 1 && (int64_t)p->h.W * p->h.H >= 8 && p->nscale <= 1024 && p->d_wave_flags;
+}
+
 size_t dense_series_elems(const xpcs_mt_plan* p)
 {
     const HostTables& h = p->h;
     const size_t K = (size_t)dense_levels(p);
     // 32-bit words: u32 level values, or FP64 frame-weighted values (2 words)
     const size_t words = p->fsnorm ? 2 : 1;
-    return h.levels.size() > K ? words * (size_t)h.levels[K].lf * (size_t)h.W * (size_t)h.H : 1;
+    const size_t series = h.levels.size() > K ? words * (size_t)h.levels[K].lf * (size_t)h.W * (size_t)h.H : 1;
+    // the first pass keeps its boundary sums in the second buffer
+    return std::max(series, dense_dot_ok(p) ? (size_t)p->nrank * (size_t)h.W * (size_t)h.H : (size_t)1);
+}
+
+template <int DPL, int K>
+static void launch_dense_dot(xpcs_mt_plan* p, hipStream_t s, int nlev_pass, uint32_t* out, uint32_t lf_out,
+                             uint32_t* redo_count)
+{
+    const HostTables& h = p->h;
+    DotArgs a{};
+    a.src = p->d_imm + p->even_off0;
+    a.step = p->even_step;
+    a.pix2c = p->d_pix2c;
+    a.npix = (uint32_t)(h.W * h.H);
+    a.n_in = (uint32_t)h.F;
+    a.dark_sum = p->d_dark_sum;
+    a.thr = p->d_thr;
+    a.nscale = (int32_t)p->nscale;
+    a.levels = p->d_levels;
+    a.nlev_pass = nlev_pass;
+    a.cap = p->d_cap;
+    a.ncap = p->nrank;
+    a.T = h.T;
+    a.tau_bnd = p->d_tau_bnd;
+    a.cap_sums = p->d_series_b;   // free during the first pass
+    a.G2 = p->d_G2;
+    a.IP = p->d_IP;
+    a.IF = p->d_IF;
+    a.pix_total = p->d_pix_total;
+    a.series_out = out;
+    a.lf_out = (out && nlev_pass == K) ? lf_out : 0u;
+    a.redo_count = redo_count;
+    a.redo_list = p->d_long_list;
+    a.wave_flags = p->d_wave_flags;
+    a.w32 = p->ipif32;
+    auto go = [&](auto waves) {
+        constexpr int W = decltype(waves)::value;
+        const unsigned grid = ((a.npix + 64 * W - 1) / (64 * W) + 7) / 8 * 8;
+        if (h.darks > 0) k_mt_dense_dot<DPL, K, true, W><<<grid, 64 * W, 0, s>>>(a);
+        else k_mt_dense_dot<DPL, K, false, W><<<grid, 64 * W, 0, s>>>(a);
+    };
+    // detectors of at most two waves per CU: single waves spread over the chip
+    if (a.npix <= 2 * 256 * 64) go(std::integral_constant<int, 1>{});
+    else go(std::integral_constant<int, DPL == 4 ? 8 : 4>{});
 }
 
 template <int DPL, int K, bool FP>
@@ -721,16 +1178,25 @@ static void run_passes(xpcs_mt_plan* p, hipStream_t s)
         const ST* in = pass == 0 ? nullptr : (pass % 2 == 1 ? sa : sb);
         if (pass == 0) {
             timer_begin(p, s, FP ? "k_mt_dense_raw_f64" : "k_mt_dense_raw");
+            // counts of evenly spaced frames: the dot-product kernel, then the
+            // FP64 one for the pixels it left
+            const uint32_t* only = nullptr;
+            if constexpr (!FP && (8 >> (K - 1)) >= 1) {
+                if (dense_dot_ok(p)) {
+                    launch_dense_dot<DPL, K>(p, s, k, out, lf_out, redo_count);
+                    only = p->d_wave_flags;
+                }
+            }
             if (p->tile_off0 >= 0)
                 k_mt_dense_f64<DPL, K, kRawTiles, FP><<<grid, 256, 0, s>>>(
                     p->d_imm, p->d_sel_off, p->tile_off0, p->tile_step, h.avg, p->d_pix2c, npd, p->d_dark_sum,
                     p->d_thr, (int32_t)p->nscale, nullptr, n_in, p->d_levels, L0, k, p->d_bnd, p->nbnd, h.T,
-                    p->d_G2, p->d_IP, p->d_IF, p->d_pix_total, out, lf_out, redo_count, p->d_long_list, fw, !FP && p->ipif32);
+                    p->d_G2, p->d_IP, p->d_IF, p->d_pix_total, out, lf_out, redo_count, p->d_long_list, fw, !FP && p->ipif32, only);
             else
                 k_mt_dense_f64<DPL, K, kRawLanes, FP><<<grid, 256, 0, s>>>(
                     p->d_imm, p->d_sel_off, 0, 0, h.avg, p->d_pix2c, npd, p->d_dark_sum, p->d_thr,
                     (int32_t)p->nscale, nullptr, n_in, p->d_levels, L0, k, p->d_bnd, p->nbnd, h.T, p->d_G2,
-                    p->d_IP, p->d_IF, p->d_pix_total, out, lf_out, redo_count, p->d_long_list, fw, !FP && p->ipif32);
+                    p->d_IP, p->d_IF, p->d_pix_total, out, lf_out, redo_count, p->d_long_list, fw, !FP && p->ipif32, only);
             timer_end(p, s);
             if constexpr (!FP) {
                 timer_begin(p, s, "k_mt_dense_exact");
@@ -744,7 +1210,7 @@ static void run_passes(xpcs_mt_plan* p, hipStream_t s)
             k_mt_dense_f64<DPL, K, kSeries, FP><<<grid, 256, 0, s>>>(
                 nullptr, nullptr, 0, 0, 1, p->d_pix2c, npd, nullptr, nullptr, 1, in, n_in, p->d_levels, L0, k,
                 nullptr, 0, h.T, p->d_G2, p->d_IP, p->d_IF, p->d_pix_total, out, lf_out, nullptr, nullptr, fw,
-                !FP && p->ipif32);
+                !FP && p->ipif32, nullptr);
             timer_end(p, s);
             if constexpr (!FP) {
                 timer_begin(p, s, "k_mt_dense_exact");
