@@ -300,7 +300,7 @@ extern "C" xpcs_status xpcs_mt_plan_destroy(xpcs_mt_plan* p)
     dfree(p->d_group_chunk_first); dfree(p->d_group_q); dfree(p->d_group_size);
     dfree(p->d_q_chunk_first); dfree(p->d_q_first_group); dfree(p->d_weight); dfree(p->d_c2pix);
     dfree(p->d_sbin_of_c); dfree(p->d_sbin_pix); dfree(p->d_imm_owned); dfree(p->d_sel_off); dfree(p->d_sel_dlen);
-    dfree(p->d_sel_frame); dfree(p->d_dark_sum); dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_off);
+    dfree(p->d_sel_frame); dfree(p->d_dark_sum); dfree(p->d_dark_avg); dfree(p->d_dark_std); dfree(p->d_dark_isum); dfree(p->d_dark_raw); dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_off);
     dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_wide_list); dfree(p->d_wave_flags); dfree(p->d_counters);
     dfree(p->d_scratch); dfree(p->d_G2); dfree(p->d_IP); dfree(p->d_IF); dfree(p->d_pix_total); dfree(p->d_fw);
     dfree(p->d_deep);
@@ -421,46 +421,44 @@ xpcs_status select_frames(const HostTables& h, int64_t n_raw, bool compressed, i
     return XPCS_OK;
 }
 
-// Dark image of the first `darks` frames (DarkImage::Compute,
-// src/xpcs/data_structure/dark_image.cpp:81-106, Welford in double) plus the
-// exact integer sums used for the n-scaled threshold of the dense path.  Dark
-// values are uint16 like every count (the reference reads int16,
-// src/xpcs/io/imm.cpp:87; equal below 32768), so the threshold's standard
-// deviation and the subtracted sums describe the same values.
-xpcs_status dense_prepare(xpcs_mt_plan* p, const uint8_t* const* dark_frames)
+xpcs_status h2d_staged(uint8_t* dst, const uint8_t* src, size_t len, hipStream_t s);
+
+// Work of earlier calls may still read the buffers an ingest overwrites.  On the
+// plan's own stream the copies queue up behind it; work that went to another
+// stream, or into a batch, is waited for.
+xpcs_status ingest_begin(xpcs_mt_plan* p)
+{
+    if (p->foreign) HIP_TRY(hipDeviceSynchronize());
+    return XPCS_OK;
+}
+
+// Dark image of the first `darks` frames and the integer form of the dense
+// path's threshold (launch_dark_image): frame i's values at base + off[i] in
+// device memory.
+xpcs_status dense_prepare(xpcs_mt_plan* p, const uint8_t* base, const std::vector<int64_t>& off)
 {
     HostTables& h = p->h;
-    const int64_t npd = (int64_t)h.W * h.H;
     p->nscale = h.darks > 0 ? h.darks : 1;
-    std::vector<int64_t> dsum((size_t)h.P, 0), thr((size_t)h.P, 0);
-    p->dark_avg.assign((size_t)npd, 0.0);
-    p->dark_std.assign((size_t)npd, 0.0);
-    if (h.darks > 0) {
+    xpcs_status st = XPCS_OK;
+    if (!p->d_dark_sum) st = dalloc(&p->d_dark_sum, (size_t)h.P);
+    if (!st && !p->d_thr) st = dalloc(&p->d_thr, (size_t)h.P);
+    if (st) return st;
+    if (h.darks == 0) {
+        launch_fill_u64(reinterpret_cast<uint64_t*>(p->d_dark_sum), (size_t)h.P, p->stream);
+        launch_fill_u64(reinterpret_cast<uint64_t*>(p->d_thr), (size_t)h.P, p->stream);
+    } else {
         if (!h.ff_det.empty())
             return fail(XPCS_ERR_UNSUPPORTED,
                         "dense path: a flat field together with dark frames has no exact integer form");
-        std::vector<int64_t> isum((size_t)npd, 0);
-        for (int i = 0; i < h.darks; i++) {
-            const uint16_t* v = reinterpret_cast<const uint16_t*>(dark_frames[i]);
-            for (int64_t j = 0; j < npd; j++) {
-                const double x = (double)v[j];
-                const double prev = p->dark_avg[(size_t)j];
-                p->dark_avg[(size_t)j] += (x - p->dark_avg[(size_t)j]) / (double)(i + 1);
-                p->dark_std[(size_t)j] += (x - prev) * (x - p->dark_avg[(size_t)j]);
-                isum[(size_t)j] += v[j];
-            }
-        }
-        for (int64_t j = 0; j < npd; j++) p->dark_std[(size_t)j] = std::sqrt(p->dark_std[(size_t)j] / h.darks);
-        for (int c = 0; c < h.P; c++) {
-            const int64_t j = h.order[(size_t)c];
-            const float t = (float)((double)h.lld + (double)h.sigma * p->dark_std[(size_t)j]);
-            dsum[(size_t)c] = isum[(size_t)j];
-            thr[(size_t)c] = (int64_t)std::floor((double)p->nscale * (double)t);
-        }
+        const size_t npd = (size_t)h.W * (size_t)h.H;
+        if (!p->d_dark_avg) st = dalloc(&p->d_dark_avg, npd);
+        if (!st && !p->d_dark_std) st = dalloc(&p->d_dark_std, npd);
+        if (!st && !p->d_dark_isum) st = dalloc(&p->d_dark_isum, npd);
+        if (st) return st;
+        launch_dark_image(p, base, off, p->stream);
     }
-    xpcs_status st = upload(&p->d_dark_sum, dsum, p->stream);
-    if (st) return st;
-    return upload(&p->d_thr, thr, p->stream);
+    HIP_TRY(hipGetLastError());
+    return XPCS_OK;
 }
 
 xpcs_status finish_selection(xpcs_mt_plan* p, const std::vector<int64_t>& sel_off,
@@ -588,6 +586,10 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
 {
     if (!p || !imm) return fail(XPCS_ERR_INVALID_ARG, "ingest_imm: NULL argument");
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     int64_t n = 0;
     int32_t comp = 0;
     xpcs_status st = xpcs_imm_index(imm, nbytes, nullptr, nullptr, nullptr, nullptr, 0, &n, &comp);
@@ -609,14 +611,28 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
             if ((int64_t)dl[(size_t)r] != (int64_t)h.W * h.H)
                 return fail(XPCS_ERR_FORMAT, "ingest_imm: uncompressed frame %lld has %u values, detector has %lld",
                             (long long)r, dl[(size_t)r], (long long)h.W * h.H);
-        std::vector<const uint8_t*> darks;
         for (int i = 0; i < h.darks; i++) {
             if (i >= n) return fail(XPCS_ERR_FORMAT, "ingest_imm: fewer frames than dark frames");
             if ((int64_t)dl[(size_t)i] != (int64_t)h.W * h.H)
                 return fail(XPCS_ERR_FORMAT, "ingest_imm: dark frame %d has the wrong size", i);
-            darks.push_back(b + off[(size_t)i]);
         }
-        st = dense_prepare(p, darks.data());
+        // the dark frames' values on the device, one after another
+        const size_t fb = (size_t)h.W * (size_t)h.H * 2;
+        std::vector<int64_t> doff;
+        if (h.darks > 0) {
+            if (fb * (size_t)h.darks > p->dark_cap) {
+                p->dark_cap = 0;
+                st = dalloc(&p->d_dark_raw, fb * (size_t)h.darks);
+                if (st) return st;
+                p->dark_cap = fb * (size_t)h.darks;
+            }
+            for (int i = 0; i < h.darks; i++) {
+                doff.push_back((int64_t)(fb * (size_t)i));
+                st = h2d_staged(p->d_dark_raw + doff.back(), b + off[(size_t)i], fb, p->stream);
+                if (st) return st;
+            }
+        }
+        st = dense_prepare(p, p->d_dark_raw, doff);
         if (st) return st;
     }
     // timestamps of every raw frame the load loop reads (SparseFilter::Apply
@@ -682,6 +698,10 @@ extern "C" xpcs_status xpcs_mt_ingest_events(xpcs_mt_plan* p, const int32_t* pix
     if (frame_off[nframes] > 0 && (!pixel || !count))
         return fail(XPCS_ERR_INVALID_ARG, "ingest_events: NULL pixel/count arrays");
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     std::vector<int64_t> sel;
     std::vector<int32_t> ofr;
     int64_t first = 0;
@@ -737,6 +757,10 @@ extern "C" xpcs_status xpcs_mt_ingest_imm_device(xpcs_mt_plan* p, const void* de
     if (!p || !dev_imm || !payload_off || !dlen || raw_frames <= 0)
         return fail(XPCS_ERR_INVALID_ARG, "ingest_imm_device: bad arguments");
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     std::vector<int64_t> sel;
     std::vector<int32_t> ofr;
     int64_t first = 0;
@@ -759,15 +783,8 @@ extern "C" xpcs_status xpcs_mt_ingest_imm_device(xpcs_mt_plan* p, const void* de
                 return fail(XPCS_ERR_FORMAT, "ingest_imm_device: dark frame %lld lies outside the buffer",
                             (long long)i);
         }
-        std::vector<std::vector<uint8_t>> dark_host((size_t)h.darks);
-        std::vector<const uint8_t*> darks;
-        for (int i = 0; i < h.darks; i++) {
-            dark_host[(size_t)i].resize((size_t)h.W * h.H * 2);
-            HIP_TRY(hipMemcpy(dark_host[(size_t)i].data(), static_cast<const uint8_t*>(dev_imm) + payload_off[i],
-                              dark_host[(size_t)i].size(), hipMemcpyDeviceToHost));
-            darks.push_back(dark_host[(size_t)i].data());
-        }
-        st = dense_prepare(p, darks.data());
+        st = dense_prepare(p, static_cast<const uint8_t*>(dev_imm),
+                           std::vector<int64_t>(payload_off, payload_off + h.darks));
         if (st) return st;
     }
     p->clock.clear();
@@ -797,6 +814,10 @@ extern "C" xpcs_status xpcs_mt_ingest_packed(xpcs_mt_plan* p, const void* words,
 {
     if (!p || (!words && nbytes)) return fail(XPCS_ERR_INVALID_ARG, "ingest_packed: NULL argument");
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     if (h.darks > 0) return fail(XPCS_ERR_INVALID_ARG, "ingest_packed: packed formats have no dark frames");
     std::vector<PackedRecord> rec;
     xpcs_status st = packed_records(words, nbytes, format, h, rec);
@@ -850,6 +871,10 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
     if (bytes_per_value != 2 && bytes_per_value != 4)
         return fail(XPCS_ERR_INVALID_ARG, "ingest_frames: values are 2 or 4 bytes, not %d", bytes_per_value);
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     if (h.darks > 0) return fail(XPCS_ERR_INVALID_ARG, "ingest_frames: raw frames have no dark frames");
     std::vector<int64_t> sel;
     std::vector<int32_t> ofr;
@@ -881,7 +906,7 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
     }
     if (st) return st;
     p->d_imm = p->d_imm_owned;
-    st = dense_prepare(p, nullptr);
+    st = dense_prepare(p, nullptr, {});
     if (st) return st;
     std::vector<int64_t> so(sel.size());
     std::vector<uint32_t> sd(sel.size(), (uint32_t)npd);
@@ -908,6 +933,10 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
     if ((!frame || !count) && row_off[(int64_t)p->h.W * p->h.H] > 0)
         return fail(XPCS_ERR_INVALID_ARG, "ingest_rows: NULL frame/count arrays");
     HostTables& h = p->h;
+    {
+        const xpcs_status sb = ingest_begin(p);
+        if (sb) return sb;
+    }
     const int64_t npd = (int64_t)h.W * h.H;
     if (row_off[0] < 0) return fail(XPCS_ERR_INVALID_ARG, "ingest_rows: row_off[0] < 0");
     for (int64_t j = 0; j < npd; j++)
@@ -1102,6 +1131,7 @@ extern "C" xpcs_status xpcs_mt_execute(xpcs_mt_plan* p, void* stream)
     xpcs_status st = prepare_execute(p);
     if (st) return st;
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : p->stream;
+    if (s != p->stream) p->foreign = true;
     enqueue_execute(p, s);
     HIP_TRY(hipGetLastError());
     p->stream_last = s;
@@ -1414,9 +1444,13 @@ extern "C" xpcs_status xpcs_mt_read_dark(xpcs_mt_plan* p, double* dark_avg, doub
 {
     if (!p) return fail(XPCS_ERR_INVALID_ARG, "read_dark: NULL plan");
     const size_t n = (size_t)p->h.W * p->h.H;
-    for (size_t i = 0; i < n; i++) {
-        if (dark_avg) dark_avg[i] = p->dark_avg.size() == n ? p->dark_avg[i] : 0.0;
-        if (dark_std) dark_std[i] = p->dark_std.size() == n ? p->dark_std[i] : 0.0;
+    double* out[2] = {dark_avg, dark_std};
+    const double* src[2] = {p->d_dark_avg, p->d_dark_std};
+    HIP_TRY(hipStreamSynchronize(p->stream));
+    for (int k = 0; k < 2; k++) {
+        if (!out[k]) continue;
+        if (src[k]) HIP_TRY(hipMemcpy(out[k], src[k], n * sizeof(double), hipMemcpyDeviceToHost));
+        else std::fill(out[k], out[k] + n, 0.0);
     }
     return XPCS_OK;
 }

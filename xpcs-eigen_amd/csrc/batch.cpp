@@ -313,6 +313,7 @@ extern "C" xpcs_status xpcs_mt_batch_add(xpcs_mt_batch* b, xpcs_mt_plan* p, int3
     if (std::find(b->plans.begin(), b->plans.end(), p) != b->plans.end())
         return fail(XPCS_ERR_INVALID_ARG, "batch_add: plan already in the batch");
     b->plans.push_back(p);
+    p->foreign = true;
     batch_release_graph(b);
     if (index) *index = (int32_t)b->plans.size() - 1;
     return XPCS_OK;

@@ -104,6 +104,7 @@ struct xpcs_mt_plan {
     hipStream_t stream = nullptr;
     hipStream_t stream_last = nullptr;   // stream of the last execute
     bool own_stream = false;
+    bool foreign = false;                // work of this plan has gone to another stream or into a batch
 
 
     // device tables
@@ -162,7 +163,11 @@ struct xpcs_mt_plan {
     int64_t nscale = 1;                  // value scale (dark frames)
     int64_t* d_dark_sum = nullptr;       // [P] per compact pixel
     int64_t* d_thr = nullptr;            // [P]
-    std::vector<double> dark_avg, dark_std;   // [W*H] (host, --darkout)
+    double* d_dark_avg = nullptr;        // [W*H] dark image, plans with dark frames (--darkout)
+    double* d_dark_std = nullptr;
+    int64_t* d_dark_isum = nullptr;      // [W*H] dark sums
+    uint8_t* d_dark_raw = nullptr;       // the dark frames of a host ingest
+    size_t dark_cap = 0;
 
     // events (pixel-major CSR over compact pixels)
     int64_t ev_cap = 0;
@@ -369,6 +374,9 @@ void launch_stream_snapshot(const StreamLaunch& a, int32_t n, const LevelParam* 
 void enqueue_execute(xpcs_mt_plan* p, hipStream_t s);
 void launch_mt_dense(xpcs_mt_plan* p, hipStream_t s, bool fsnorm);
 void launch_side_dense_raw(xpcs_mt_plan* p, hipStream_t s);
+// dark image (mean, deviation), dark sums and thresholds from the dark frames
+// at base + off[i] in device memory
+void launch_dark_image(xpcs_mt_plan* p, const uint8_t* base, const std::vector<int64_t>& off, hipStream_t s);
 void launch_normalize(xpcs_mt_plan* p, hipStream_t s);
 void launch_ref_f32(xpcs_mt_plan* p, hipStream_t s, float* G2, float* IP, float* IF);
 

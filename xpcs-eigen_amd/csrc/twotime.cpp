@@ -152,6 +152,7 @@ extern "C" xpcs_status xpcs_mt_twotime(xpcs_mt_plan* p, const xpcs_tt_desc* d, v
     HostTables& h = p->h;
     const int32_t F = h.F;
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : p->stream;
+    if (s != p->stream) p->foreign = true;
     // the previous results may still be read by work queued on another stream
     HIP_TRY(hipStreamSynchronize(p->stream));
     recycle(p);
