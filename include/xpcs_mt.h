@@ -164,6 +164,8 @@ xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* plan, const void* imm, size_t nbyte
  * dlen[i] describe raw frame i (byte offset of its payload in dev_imm and its
  * entry count, as Imm::NextFrames reads them); compressed != 0 selects the
  * sparse layout.  The device buffer must stay valid until execute returns.
+ * Work queued on the device before the call (what fills the buffer, on any
+ * stream) is waited for.
  */
 xpcs_status xpcs_mt_ingest_imm_device(xpcs_mt_plan* plan, const void* dev_imm, size_t nbytes,
                                       const int64_t* payload_off, const uint32_t* dlen,

@@ -757,10 +757,9 @@ extern "C" xpcs_status xpcs_mt_ingest_imm_device(xpcs_mt_plan* p, const void* de
     if (!p || !dev_imm || !payload_off || !dlen || raw_frames <= 0)
         return fail(XPCS_ERR_INVALID_ARG, "ingest_imm_device: bad arguments");
     HostTables& h = p->h;
-    {
-        const xpcs_status sb = ingest_begin(p);
-        if (sb) return sb;
-    }
+    // the caller's frames may still be written on another stream (its default
+    // stream, say): everything queued on the device before this call finishes first
+    HIP_TRY(hipDeviceSynchronize());
     std::vector<int64_t> sel;
     std::vector<int32_t> ofr;
     int64_t first = 0;
