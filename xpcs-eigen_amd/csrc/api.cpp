@@ -54,6 +54,44 @@ static xpcs_status upload(T** p, const std::vector<T>& v, hipStream_t s)
     return XPCS_OK;
 }
 
+// One device allocation for everything a plan holds from its creation: the
+// tables first (one host image, one copy), then the buffers.  Thirty separate
+// allocations and copies took 2 ms of opening a 256 x 256 stream.
+class Arena {
+public:
+    template <typename T>
+    void table(T** p, const std::vector<T>& v)
+    {
+        const size_t off = aligned(image_.size());
+        image_.resize(off + std::max<size_t>(v.size(), 1) * sizeof(T));
+        if (!v.empty()) std::memcpy(image_.data() + off, v.data(), v.size() * sizeof(T));
+        tables_.push_back({reinterpret_cast<void**>(p), off});
+    }
+    template <typename T>
+    void buffer(T** p, size_t n)
+    {
+        buffers_.push_back({reinterpret_cast<void**>(p), bytes_});
+        bytes_ += aligned(std::max<size_t>(n, 1) * sizeof(T));
+    }
+    xpcs_status commit(uint8_t** block, hipStream_t s)
+    {
+        const size_t head = aligned(image_.size());
+        xpcs_status st = dalloc(block, head + bytes_);
+        if (st) return st;
+        for (auto& t : tables_) *t.first = *block + t.second;
+        for (auto& b : buffers_) *b.first = *block + head + b.second;
+        if (!image_.empty() && hipMemcpyAsync(*block, image_.data(), image_.size(), hipMemcpyHostToDevice, s) != hipSuccess)
+            return fail(XPCS_ERR_HIP, "plan_create: table upload failed");
+        return XPCS_OK;
+    }
+
+private:
+    static size_t aligned(size_t n) { return (n + 255) & ~(size_t)255; }
+    std::vector<uint8_t> image_;
+    std::vector<std::pair<void**, size_t>> tables_, buffers_;
+    size_t bytes_ = 0;
+};
+
 template <typename T>
 static void dfree(T*& p)
 {
@@ -145,9 +183,10 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
             return st;                \
         }                             \
     } while (0)
-    TRY(upload(&p->d_pix2c, h.pix2c, s));
-    TRY(upload(&p->d_taus, h.taus, s));
-    TRY(upload(&p->d_levels, h.levels, s));
+    Arena mem;
+    mem.table(&p->d_pix2c, h.pix2c);
+    mem.table(&p->d_taus, h.taus);
+    mem.table(&p->d_levels, h.levels);
     {
         // distinct frame boundaries of the IP/IF prefix sums, (lf - tau') 2^L,
         // tau' 2^L and lf 2^L, each tau's indices among them, and per frame
@@ -191,45 +230,45 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
             const uint32_t r = q.z + (uint32_t)__builtin_popcountll(bits & (~0ull >> (63 - (f & 63))));
             words_ok = r == rank[(size_t)f];
         }
-        TRY(upload(&p->d_tau_bnd, tj, s));
+        mem.table(&p->d_tau_bnd, tj);
         std::vector<int32_t> cap(b);
         cap.push_back(INT32_MAX);
-        TRY(upload(&p->d_cap, cap, s));
-        TRY(upload(&p->d_frame_rank, rank, s));
+        mem.table(&p->d_cap, cap);
+        mem.table(&p->d_frame_rank, rank);
         if (words_ok && nw > 0) {
-            TRY(upload(&p->d_rank_words, words, s));
+            mem.table(&p->d_rank_words, words);
             p->nrank_words = nw;
         }
     }
-    TRY(upload(&p->d_chunks, h.chunks, s));
-    TRY(upload(&p->d_group_chunk_first, h.group_chunk_first, s));
-    TRY(upload(&p->d_group_q, h.group_q, s));
-    TRY(upload(&p->d_group_size, gsize, s));
-    TRY(upload(&p->d_q_chunk_first, qchunk, s));
-    TRY(upload(&p->d_q_first_group, h.q_first_group, s));
-    TRY(upload(&p->d_c2pix, h.order, s));
-    TRY(upload(&p->d_sbin_of_c, h.sbin_of_c, s));
-    if (!h.weight.empty()) TRY(upload(&p->d_weight, h.weight, s));
+    mem.table(&p->d_chunks, h.chunks);
+    mem.table(&p->d_group_chunk_first, h.group_chunk_first);
+    mem.table(&p->d_group_q, h.group_q);
+    mem.table(&p->d_group_size, gsize);
+    mem.table(&p->d_q_chunk_first, qchunk);
+    mem.table(&p->d_q_first_group, h.q_first_group);
+    mem.table(&p->d_c2pix, h.order);
+    mem.table(&p->d_sbin_of_c, h.sbin_of_c);
+    if (!h.weight.empty()) mem.table(&p->d_weight, h.weight);
     const size_t PT = (size_t)h.P * (size_t)h.T;
-    TRY(dalloc(&p->d_G2, PT));
-    TRY(dalloc(&p->d_IP, PT));
-    TRY(dalloc(&p->d_IF, PT));
-    TRY(dalloc(&p->d_pix_total, (size_t)h.P));
-    TRY(dalloc(&p->d_part, std::max<size_t>(1, h.chunks.size() * (size_t)h.T)));
-    TRY(dalloc(&p->d_g2s, std::max<size_t>(1, (size_t)h.ngroups * h.T)));
-    TRY(dalloc(&p->d_g2, std::max<size_t>(1, (size_t)h.nq * h.T)));
-    TRY(dalloc(&p->d_se, std::max<size_t>(1, (size_t)h.nq * h.T)));
-    TRY(dalloc(&p->d_off, (size_t)std::max<int64_t>(h.P, (int64_t)h.W * h.H) + 1));
+    mem.buffer(&p->d_G2, PT);
+    mem.buffer(&p->d_IP, PT);
+    mem.buffer(&p->d_IF, PT);
+    mem.buffer(&p->d_pix_total, (size_t)h.P);
+    mem.buffer(&p->d_part, std::max<size_t>(1, h.chunks.size() * (size_t)h.T));
+    mem.buffer(&p->d_g2s, std::max<size_t>(1, (size_t)h.ngroups * h.T));
+    const size_t QT = std::max<size_t>(1, (size_t)h.nq * h.T);
+    mem.buffer(&p->d_stat, sizeof(RunStatus) / sizeof(int64_t) + 2 * QT);   // status, g2, stderr: one copy reads them
+    mem.buffer(&p->d_off, (size_t)std::max<int64_t>(h.P, (int64_t)h.W * h.H) + 1);
     {
         const int64_t npd = (int64_t)h.W * h.H;
         std::vector<uint32_t> bits((size_t)(npd / 32 + 1), 0u);
         for (int64_t i = 0; i < npd; i++)
             if (h.pix2c[(size_t)i] >= 0) bits[(size_t)(i >> 5)] |= 1u << (i & 31);
-        TRY(upload(&p->d_mapped, bits, s));
+        mem.table(&p->d_mapped, bits);
     }
-    TRY(dalloc(&p->d_long_list, (size_t)h.P));
-    TRY(dalloc(&p->d_mid_list, (size_t)h.P));
-    TRY(dalloc(&p->d_counters, 8));
+    mem.buffer(&p->d_long_list, (size_t)h.P);
+    mem.buffer(&p->d_mid_list, (size_t)h.P);
+    mem.buffer(&p->d_counters, 8);
     {
         // level-0 prefix boundaries of the dense streaming path
         std::vector<int4> bnd;
@@ -243,7 +282,7 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
             return a.x != b.x ? a.x < b.x : a.y < b.y;
         });
         p->nbnd = (int32_t)bnd.size();
-        TRY(upload(&p->d_bnd, bnd, s));
+        mem.table(&p->d_bnd, bnd);
     }
     p->fsnorm = (h.flags & XPCS_MT_NORMALIZE_BY_FRAMESUM) != 0;
     if (h.flags & (XPCS_MT_SIDE_STATS | XPCS_MT_NORMALIZE_BY_FRAMESUM)) {
@@ -251,27 +290,23 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
             xpcs_mt_plan_destroy(p);
             return fail(XPCS_ERR_UNSUPPORTED, "plan: side statistics need S <= 4096 and F*S <= 2^26");
         }
-        TRY(dalloc(&p->d_fs, (size_t)h.F * h.ns));
+        mem.buffer(&p->d_fs, (size_t)h.F * h.ns);
         // static bin (1..S, 0 unmapped) per raster pixel, one byte when S < 256:
         // one small gather per sparse event instead of the pixel's row id and
         // then its bin
         if (h.ns < 256) {
             std::vector<uint8_t> sbp((size_t)h.W * h.H, 0);
             for (int c = 0; c < h.P; c++) sbp[(size_t)h.order[(size_t)c]] = (uint8_t)h.sbin_of_c[(size_t)c];
-            uint8_t* d = nullptr;
-            TRY(upload(&d, sbp, s));
-            p->d_sbin_pix = d;
+            mem.table(reinterpret_cast<uint8_t**>(&p->d_sbin_pix), sbp);
             p->sbin_pix_bytes = 1;
         } else {
             std::vector<uint16_t> sbp((size_t)h.W * h.H, 0);
             for (int c = 0; c < h.P; c++) sbp[(size_t)h.order[(size_t)c]] = (uint16_t)h.sbin_of_c[(size_t)c];
-            uint16_t* d = nullptr;
-            TRY(upload(&d, sbp, s));
-            p->d_sbin_pix = d;
+            mem.table(reinterpret_cast<uint16_t**>(&p->d_sbin_pix), sbp);
             p->sbin_pix_bytes = 2;
         }
     }
-    if (p->fsnorm) TRY(dalloc(&p->d_fw, (size_t)h.F));
+    if (p->fsnorm) mem.buffer(&p->d_fw, (size_t)h.F);
     // dense-row scratch (allocated by the first execute that needs it): one row
     // of F 64-bit values per resident workgroup
     {
@@ -282,6 +317,9 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
         // one wavefront per pixel: more, smaller workgroups (4 GiB of rows)
         if (p->fsnorm) p->long_blocks = (int)std::min<size_t>(8192, std::max<size_t>(1, 4 * budget / per));
     }
+    TRY(mem.commit(&p->d_arena, s));
+    p->d_g2 = reinterpret_cast<double*>(p->d_stat + sizeof(RunStatus) / sizeof(int64_t));
+    p->d_se = p->d_g2 + QT;
     if (hipMemsetAsync(p->d_counters, 0, 32, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         xpcs_mt_plan_destroy(p);
@@ -296,15 +334,11 @@ extern "C" xpcs_status xpcs_mt_plan_destroy(xpcs_mt_plan* p)
 {
     if (!p) return XPCS_OK;
     if (p->stream) (void)hipStreamSynchronize(p->stream);
-    dfree(p->d_pix2c); dfree(p->d_mapped); dfree(p->d_taus); dfree(p->d_levels); dfree(p->d_tau_bnd); dfree(p->d_frame_rank); dfree(p->d_rank_words); dfree(p->d_chunks);
-    dfree(p->d_group_chunk_first); dfree(p->d_group_q); dfree(p->d_group_size);
-    dfree(p->d_q_chunk_first); dfree(p->d_q_first_group); dfree(p->d_weight); dfree(p->d_c2pix);
-    dfree(p->d_sbin_of_c); dfree(p->d_sbin_pix); dfree(p->d_imm_owned); dfree(p->d_sel_off); dfree(p->d_sel_dlen);
-    dfree(p->d_sel_frame); dfree(p->d_dark_sum); dfree(p->d_dark_avg); dfree(p->d_dark_std); dfree(p->d_dark_isum); dfree(p->d_dark_raw); dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_off);
-    dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum); dfree(p->d_rows); dfree(p->d_long_list); dfree(p->d_mid_list); dfree(p->d_wide_list); dfree(p->d_wave_flags); dfree(p->d_counters);
-    dfree(p->d_scratch); dfree(p->d_G2); dfree(p->d_IP); dfree(p->d_IF); dfree(p->d_pix_total); dfree(p->d_fw);
-    dfree(p->d_deep);
-    dfree(p->d_part); dfree(p->d_g2s); dfree(p->d_g2); dfree(p->d_se); dfree(p->d_fs); dfree(p->d_series_a); dfree(p->d_series_b); dfree(p->d_bnd); dfree(p->d_cap);
+    dfree(p->d_arena); dfree(p->d_sel);
+    dfree(p->d_imm_owned); dfree(p->d_dark_sum); dfree(p->d_dark_avg); dfree(p->d_dark_std); dfree(p->d_dark_isum); dfree(p->d_dark_raw);
+    dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum);
+    dfree(p->d_rows); dfree(p->d_wide_list); dfree(p->d_wave_flags); dfree(p->d_scratch); dfree(p->d_deep); dfree(p->d_series_a);
+    dfree(p->d_series_b);
     for (auto& t : p->pending) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     for (auto e : p->event_pool) (void)hipEventDestroy(e);
     twotime_release(p);
@@ -464,13 +498,26 @@ xpcs_status dense_prepare(xpcs_mt_plan* p, const uint8_t* base, const std::vecto
 xpcs_status finish_selection(xpcs_mt_plan* p, const std::vector<int64_t>& sel_off,
                              const std::vector<uint32_t>& sel_dlen, const std::vector<int32_t>& sel_frame)
 {
-    p->nsel = (int64_t)sel_off.size();
-    xpcs_status st = upload(&p->d_sel_off, sel_off, p->stream);
-    if (st) return st;
-    st = upload(&p->d_sel_dlen, sel_dlen, p->stream);
-    if (st) return st;
-    st = upload(&p->d_sel_frame, sel_frame, p->stream);
-    if (st) return st;
+    const size_t n = sel_off.size();
+    p->nsel = (int64_t)n;
+    // offsets, lengths and output frames in one kept buffer, one copy
+    const size_t bytes = std::max<size_t>(n, 1) * (sizeof(int64_t) + sizeof(uint32_t) + sizeof(int32_t));
+    if (bytes > p->sel_cap) {
+        p->sel_cap = 0;
+        const xpcs_status st = dalloc(&p->d_sel, bytes);
+        if (st) return st;
+        p->sel_cap = bytes;
+    }
+    p->d_sel_off = reinterpret_cast<int64_t*>(p->d_sel);
+    p->d_sel_dlen = reinterpret_cast<uint32_t*>(p->d_sel_off + n);
+    p->d_sel_frame = reinterpret_cast<int32_t*>(p->d_sel_dlen + n);
+    p->h_sel.resize(bytes);
+    if (n) {
+        std::memcpy(p->h_sel.data(), sel_off.data(), n * sizeof(int64_t));
+        std::memcpy(p->h_sel.data() + n * 8, sel_dlen.data(), n * sizeof(uint32_t));
+        std::memcpy(p->h_sel.data() + n * 12, sel_frame.data(), n * sizeof(int32_t));
+        HIP_TRY(hipMemcpyAsync(p->d_sel, p->h_sel.data(), n * 16, hipMemcpyHostToDevice, p->stream));
+    }
     int64_t raw = 0;
     for (uint32_t d : sel_dlen) raw += d;
     p->raw_events = raw;
@@ -490,34 +537,63 @@ struct StagePool {
     size_t bytes = 0;
 };
 
+constexpr size_t kStage = size_t(32) << 20;
+
+// The pool of the current device (lives until the process ends).
 StagePool& stage_pool()
 {
-    static StagePool pool;   // lives until the process ends
-    return pool;
+    static StagePool pools[16];
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    return pools[dev & 15];
+}
+
+// The pool's buffers and events, made on first use (sp.mu held).
+xpcs_status stage_ready(StagePool& sp)
+{
+    if (sp.buf[0]) return XPCS_OK;
+    for (int i = 0; i < 2; i++) {
+        if (hipHostMalloc(reinterpret_cast<void**>(&sp.buf[i]), kStage, hipHostMallocDefault) != hipSuccess ||
+            hipEventCreateWithFlags(&sp.done[i], hipEventDisableTiming) != hipSuccess) {
+            for (int j = 0; j <= i; j++) {
+                if (sp.buf[j]) (void)hipHostFree(sp.buf[j]);
+                sp.buf[j] = nullptr;
+            }
+            return fail(XPCS_ERR_NOMEM, "pinned staging of %zu bytes failed", kStage);
+        }
+    }
+    sp.bytes = kStage;
+    return XPCS_OK;
+}
+
+// memcpy over several threads (a thread that cannot be started leaves its part
+// to this one).
+void parallel_copy(uint8_t* dst, const uint8_t* src, size_t n)
+{
+    const unsigned nthreads = n < (size_t(1) << 20) ? 1u : std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    const size_t per = (n + nthreads - 1) / nthreads;
+    std::thread pool[8];
+    for (unsigned t = 1; t < nthreads && t * per < n; t++) {
+        const size_t len = std::min(per, n - t * per);
+        try {
+            pool[t] = std::thread([=] { std::memcpy(dst + t * per, src + t * per, len); });
+        } catch (...) {
+            std::memcpy(dst + t * per, src + t * per, len);
+        }
+    }
+    std::memcpy(dst, src, std::min(per, n));
+    for (auto& th : pool)
+        if (th.joinable()) th.join();
 }
 
 xpcs_status h2d_staged(uint8_t* dst, const uint8_t* src, size_t len, hipStream_t s)
 {
-    constexpr size_t kStage = size_t(32) << 20;
     if (len == 0) return XPCS_OK;
     StagePool& sp = stage_pool();
     std::lock_guard<std::mutex> lk(sp.mu);
-    if (!sp.buf[0]) {
-        for (int i = 0; i < 2; i++) {
-            if (hipHostMalloc(reinterpret_cast<void**>(&sp.buf[i]), kStage, hipHostMallocDefault) != hipSuccess ||
-                hipEventCreateWithFlags(&sp.done[i], hipEventDisableTiming) != hipSuccess) {
-                for (int j = 0; j <= i; j++) {
-                    if (sp.buf[j]) (void)hipHostFree(sp.buf[j]);
-                    sp.buf[j] = nullptr;
-                }
-                return fail(XPCS_ERR_NOMEM, "ingest: pinned staging of %zu bytes failed", kStage);
-            }
-        }
-        sp.bytes = kStage;
-    }
-    const unsigned nthreads = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    xpcs_status st = stage_ready(sp);
+    if (st) return st;
     int b = 0;
-    xpcs_status st = XPCS_OK;
     bool issued[2] = {false, false};
     for (size_t off = 0; off < len && !st; off += sp.bytes, b ^= 1) {
         const size_t n = std::min(sp.bytes, len - off);
@@ -525,15 +601,8 @@ xpcs_status h2d_staged(uint8_t* dst, const uint8_t* src, size_t len, hipStream_t
             st = fail(XPCS_ERR_HIP, "ingest: staging copy failed");
             break;
         }
-        // parallel host copy into the pinned buffer
-        uint8_t* stage = sp.buf[b];
-        const size_t per = (n + nthreads - 1) / nthreads;
-        std::vector<std::thread> pool;
-        for (unsigned t = 1; t < nthreads && t * per < n; t++)
-            pool.emplace_back([=] { std::memcpy(stage + t * per, src + off + t * per, std::min(per, n - t * per)); });
-        std::memcpy(stage, src + off, std::min(per, n));
-        for (auto& th : pool) th.join();
-        if (hipMemcpyAsync(dst + off, stage, n, hipMemcpyHostToDevice, s) != hipSuccess ||
+        parallel_copy(sp.buf[b], src + off, n);   // into the pinned buffer
+        if (hipMemcpyAsync(dst + off, sp.buf[b], n, hipMemcpyHostToDevice, s) != hipSuccess ||
             hipEventRecord(sp.done[b], s) != hipSuccess)
             st = fail(XPCS_ERR_HIP, "ingest: host-to-device copy failed");
         issued[b] = true;
@@ -581,6 +650,46 @@ void dense_tiling(xpcs_mt_plan* p, const std::vector<int64_t>& so, const uint8_t
 }
 
 }  // namespace
+
+namespace xpcs {
+
+// Device results to pageable host memory, after the work queued on s.  Large
+// ones come through the pinned buffers a piece at a time, one piece on the
+// link while threads copy the other out (a plain copy ran at 13 GB/s, most of
+// it first-touch page faults of the caller's array on one thread).
+xpcs_status d2h_staged(void* dst, const void* src, size_t len, hipStream_t s)
+{
+    constexpr size_t kPiece = size_t(8) << 20;
+    if (len == 0) return XPCS_OK;
+    if (len < (size_t(2) << 20)) {
+        HIP_TRY(hipMemcpyAsync(dst, src, len, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return XPCS_OK;
+    }
+    StagePool& sp = stage_pool();
+    std::lock_guard<std::mutex> lk(sp.mu);
+    xpcs_status st = stage_ready(sp);
+    if (st) return st;
+    uint8_t* d = static_cast<uint8_t*>(dst);
+    const uint8_t* q = static_cast<const uint8_t*>(src);
+    const size_t pieces = (len + kPiece - 1) / kPiece;
+    auto issue = [&](size_t k) {
+        const size_t off = k * kPiece, n = std::min(kPiece, len - off);
+        if (hipMemcpyAsync(sp.buf[k & 1], q + off, n, hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipEventRecord(sp.done[k & 1], s) != hipSuccess)
+            st = fail(XPCS_ERR_HIP, "read: device-to-host copy failed");
+    };
+    issue(0);
+    for (size_t k = 0; k < pieces && !st; k++) {
+        if (k + 1 < pieces) issue(k + 1);
+        if (hipEventSynchronize(sp.done[k & 1]) != hipSuccess) st = fail(XPCS_ERR_HIP, "read: device-to-host copy failed");
+        if (!st) parallel_copy(d + k * kPiece, sp.buf[k & 1], std::min(kPiece, len - k * kPiece));
+    }
+    if (st) (void)hipStreamSynchronize(s);   // nothing may still write the pool
+    return st;
+}
+
+}  // namespace xpcs
 
 extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size_t nbytes)
 {
@@ -1138,19 +1247,23 @@ extern "C" xpcs_status xpcs_mt_execute(xpcs_mt_plan* p, void* stream)
     return XPCS_OK;
 }
 
-static xpcs_status sync_and_check(xpcs_mt_plan* p)
+// Waits for the last execute; its errors and event count, and g2 / stderr when asked for.
+static xpcs_status sync_and_check(xpcs_mt_plan* p, double* g2 = nullptr, double* se = nullptr)
 {
+    // the status record and, right behind it, g2 and stderr in one copy
+    const size_t n = sizeof(RunStatus) + (g2 || se ? 2 * (size_t)p->h.nq * p->h.T * sizeof(double) : 0);
+    p->h_result.resize(n);
     hipStream_t s = p->stream_last ? p->stream_last : p->stream;
+    HIP_TRY(hipMemcpyAsync(p->h_result.data(), p->d_stat, n, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     collect_timers(p);
-    uint32_t cnt[2] = {0, 0};
-    HIP_TRY(hipMemcpy(cnt, p->d_counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    if (cnt[1] & 1u) return fail(XPCS_ERR_RANGE, "execute: an IMM pixel index lies outside the detector");
-    if (p->mode == 1) {
-        int64_t e = 0;
-        HIP_TRY(hipMemcpy(&e, p->d_off + p->nrows, sizeof(e), hipMemcpyDeviceToHost));
-        p->events = e;
-    }
+    RunStatus r;
+    std::memcpy(&r, p->h_result.data(), sizeof(r));
+    if (r.errors & 1u) return fail(XPCS_ERR_RANGE, "execute: an IMM pixel index lies outside the detector");
+    if (p->mode == 1) p->events = r.events;
+    const size_t half = (size_t)p->h.nq * p->h.T * sizeof(double);
+    if (g2) std::memcpy(g2, p->h_result.data() + sizeof(r), half);
+    if (se) std::memcpy(se, p->h_result.data() + sizeof(r) + half, half);
     return XPCS_OK;
 }
 
@@ -1167,8 +1280,7 @@ static xpcs_status read_ipif(xpcs_mt_plan* p, const int64_t* d, int64_t* out)
 {
     const size_t n = (size_t)p->h.P * p->h.T;
     if (!p->ipif32) {
-        HIP_TRY(hipMemcpy(out, d, n * sizeof(int64_t), hipMemcpyDeviceToHost));
-        return XPCS_OK;
+        return d2h_staged(out, d, n * sizeof(int64_t), p->stream);
     }
     std::vector<uint32_t> w(2 * n);
     std::vector<uint64_t> tot((size_t)p->h.P);
@@ -1217,7 +1329,10 @@ extern "C" xpcs_status xpcs_mt_read_sums_i64(xpcs_mt_plan* p, int64_t* G2, int64
     xpcs_status st = sync_and_check(p);
     if (st) return st;
     const size_t n = (size_t)p->h.P * p->h.T * sizeof(int64_t);
-    if (G2) HIP_TRY(hipMemcpy(G2, p->d_G2, n, hipMemcpyDeviceToHost));
+    if (G2) {
+        st = d2h_staged(G2, p->d_G2, n, p->stream);
+        if (st) return st;
+    }
     if (IP && (st = read_ipif(p, p->d_IP, IP))) return st;
     if (IF && (st = read_ipif(p, p->d_IF, IF))) return st;
     return XPCS_OK;
@@ -1249,10 +1364,7 @@ extern "C" xpcs_status xpcs_mt_read_g2(xpcs_mt_plan* p, double* g2, double* se)
 {
     if (!p) return fail(XPCS_ERR_INVALID_ARG, "read_g2: NULL plan");
     if (!p->executed && !p->normalized) return fail(XPCS_ERR_STATE, "read_g2: execute first");
-    if (p->executed) {
-        xpcs_status st = sync_and_check(p);
-        if (st) return st;
-    }
+    if (p->executed) return sync_and_check(p, g2, se);
     const size_t n = (size_t)p->h.nq * p->h.T * sizeof(double);
     if (g2) HIP_TRY(hipMemcpy(g2, p->d_g2, n, hipMemcpyDeviceToHost));
     if (se) HIP_TRY(hipMemcpy(se, p->d_se, n, hipMemcpyDeviceToHost));

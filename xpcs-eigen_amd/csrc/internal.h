@@ -82,6 +82,14 @@ struct TransposeShape {
     int32_t nblk = 1;     // chunks
 };
 
+// What a run leaves beside its results (written by the last normalisation kernel).
+struct RunStatus {
+    int64_t events;      // level-0 events of the transposed rows
+    uint32_t errors;     // error flags of the transpose
+    uint32_t pad;
+};
+static_assert(sizeof(RunStatus) % sizeof(int64_t) == 0, "the results follow it");
+
 struct KernelTimer {
     std::string name;
     hipEvent_t a, b;
@@ -156,7 +164,9 @@ struct xpcs_mt_plan {
     int64_t* d_sel_off = nullptr;        // payload byte offset per selected raw frame
     uint32_t* d_sel_dlen = nullptr;
     int32_t* d_sel_frame = nullptr;      // output frame per selected raw frame
-    int64_t sel_cap = 0;
+    uint8_t* d_sel = nullptr;            // holds the three
+    size_t sel_cap = 0;
+    std::vector<uint8_t> h_sel;          // their host image
     int64_t raw_events = 0;              // sum of dlen over selected frames (sparse)
     std::vector<double> clock, ticks;    // timestamps of the data frames (host)
     // dense ingest
@@ -236,6 +246,9 @@ struct xpcs_mt_plan {
     uint64_t* d_pix_total = nullptr;     // [P] sum of level-0 values
     xpcs::NormPartial* d_part = nullptr; // [nchunks][T]
     double* d_g2s = nullptr;             // [ngroups][T]
+    int64_t* d_stat = nullptr;           // RunStatus, g2 and stderr, contiguous
+    std::vector<uint8_t> h_result;       // host copy of them
+    uint8_t* d_arena = nullptr;          // tables and buffers of the plan's creation
     double* d_g2 = nullptr;              // [T][Q]
     double* d_se = nullptr;              // [T][Q]
     // side statistics
@@ -309,6 +322,9 @@ struct NormOut {
     double* g2s;
     double* g2;
     double* se;
+    RunStatus* stat;            // NULL: not written
+    const uint32_t* counters;   // what it is taken from
+    const int64_t* events;
 };
 NormOut plan_norm_out(xpcs_mt_plan* p);
 void launch_normalize_sums(xpcs_mt_plan* p, hipStream_t s, int32_t t0, int32_t t1, int32_t S,
@@ -342,6 +358,7 @@ int tt_diag_segments(int32_t F);
 void launch_tt_diag(xpcs_mt_plan* p, double* C, int32_t F, int32_t wsize, int32_t total, double rescale,
                     double* partial, double* g2full, double* g2part, hipStream_t s);
 void twotime_release(xpcs_mt_plan* p);
+xpcs_status d2h_staged(void* dst, const void* src, size_t len, hipStream_t s);
 
 // online multi-tau (k_stream.hip)
 constexpr int kStreamChunk = 64;   // frames per update launch

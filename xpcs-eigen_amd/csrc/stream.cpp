@@ -37,6 +37,7 @@ struct xpcs_mt_stream {
     hipEvent_t copied = nullptr; // the last staging copy has been read
     bool copy_pending = false;
     TauParam* d_taus_snap = nullptr;
+    uint32_t* state = nullptr;   // one block: acc, total, win, head, pend, tile, d_taus_snap
     hipEvent_t done = nullptr;
     int32_t snap_n = 0;          // frames of the newest snapshot enqueued
     int32_t snap_T = 0;
@@ -142,21 +143,22 @@ extern "C" xpcs_status xpcs_mt_stream_open(const xpcs_mt_desc* desc, int32_t max
     s->d2 = 2 * h.dpl;
     s->nlev = (int32_t)h.levels.size();
     const size_t P = (size_t)h.P, L = (size_t)s->nlev, D2 = (size_t)s->d2;
-    if (!st) st = salloc(&s->win, L * D2 * P);
-    if (!st) st = salloc(&s->head, L * D2 * P);
-    if (!st) st = salloc(&s->acc, L * D2 * P);
-    if (!st) st = salloc(&s->pend, L * P);
-    if (!st) st = salloc(&s->total, P);
-    if (!st) st = salloc(&s->tile, (size_t)kStreamChunk * P);
-    if (!st) st = salloc(&s->d_taus_snap, (size_t)h.T);
+    // 64-bit arrays first; the block is cleared by one launch
+    const size_t words = 2 * (L * D2 * P) + 2 * P + 2 * (L * D2 * P) + L * P + (size_t)kStreamChunk * P;
+    const size_t tau_words = (size_t)h.T * sizeof(TauParam) / sizeof(uint32_t);
+    st = salloc(&s->state, words + tau_words + 4);
+    if (!st) {
+        s->acc = reinterpret_cast<uint64_t*>(s->state);
+        s->total = s->acc + L * D2 * P;
+        s->win = reinterpret_cast<uint32_t*>(s->total + P);
+        s->head = s->win + L * D2 * P;
+        s->pend = s->head + L * D2 * P;
+        s->tile = s->pend + L * P;
+        s->d_taus_snap = reinterpret_cast<TauParam*>(s->tile + (size_t)kStreamChunk * P);
+    }
     hipStream_t q = s->plan->stream;
     if (!st) {
-        launch_fill_u32(s->win, L * D2 * P, q);
-        launch_fill_u32(s->head, L * D2 * P, q);
-        launch_fill_u64(s->acc, L * D2 * P, q);
-        launch_fill_u32(s->pend, L * P, q);
-        launch_fill_u64(s->total, P, q);
-        launch_fill_u32(s->tile, (size_t)kStreamChunk * P, q);
+        launch_fill_u32(s->state, words, q);
         launch_fill_u32(s->plan->d_counters, 8, q);
         if (hipEventCreateWithFlags(&s->done, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&s->copied, hipEventDisableTiming) != hipSuccess ||
@@ -324,25 +326,31 @@ extern "C" xpcs_status xpcs_mt_stream_poll(xpcs_mt_stream* s, int32_t* frames_do
     return XPCS_OK;
 }
 
-static xpcs_status stream_wait(xpcs_mt_stream* s)
+// Waits for the newest snapshot; its errors, and g2 / stderr when asked for.
+static xpcs_status stream_wait(xpcs_mt_stream* s, double* g2 = nullptr, double* se = nullptr)
 {
     if (s->snap_T <= 0) return fail(XPCS_ERR_STATE, "stream: no snapshot taken");
-    HIP_TRY(hipStreamSynchronize(s->plan->stream));
+    xpcs_mt_plan* p = s->plan;
+    // status record, g2 and stderr (at the maximum schedule's size) in one copy
+    const size_t half = (size_t)p->h.nq * p->h.T * sizeof(double);
+    p->h_result.resize(sizeof(RunStatus) + (g2 || se ? 2 * half : 0));
+    HIP_TRY(hipMemcpyAsync(p->h_result.data(), p->d_stat, p->h_result.size(), hipMemcpyDeviceToHost, p->stream));
+    HIP_TRY(hipStreamSynchronize(p->stream));
     s->done_n = s->snap_n;
-    uint32_t cnt[2] = {0, 0};
-    HIP_TRY(hipMemcpy(cnt, s->plan->d_counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    if (cnt[1] & 1u) return fail(XPCS_ERR_RANGE, "stream: an IMM pixel index lies outside the detector");
+    RunStatus r;
+    std::memcpy(&r, p->h_result.data(), sizeof(r));
+    if (r.errors & 1u) return fail(XPCS_ERR_RANGE, "stream: an IMM pixel index lies outside the detector");
+    const size_t n = (size_t)s->snap_T * p->h.nq * sizeof(double);
+    if (g2) std::memcpy(g2, p->h_result.data() + sizeof(r), n);
+    if (se) std::memcpy(se, p->h_result.data() + sizeof(r) + half, n);
     return XPCS_OK;
 }
 
 extern "C" xpcs_status xpcs_mt_stream_read_g2(xpcs_mt_stream* s, double* g2, double* se, int32_t* taus)
 {
     if (!s) return fail(XPCS_ERR_INVALID_ARG, "stream_read_g2: NULL stream");
-    xpcs_status st = stream_wait(s);
+    const xpcs_status st = stream_wait(s, g2, se);
     if (st) return st;
-    const size_t n = (size_t)s->snap_T * s->plan->h.nq * sizeof(double);
-    if (g2) HIP_TRY(hipMemcpy(g2, s->plan->d_g2, n, hipMemcpyDeviceToHost));
-    if (se) HIP_TRY(hipMemcpy(se, s->plan->d_se, n, hipMemcpyDeviceToHost));
     if (taus) *taus = s->snap_T;
     return XPCS_OK;
 }
@@ -365,8 +373,7 @@ extern "C" xpcs_status xpcs_mt_stream_close(xpcs_mt_stream* s)
 {
     if (!s) return XPCS_OK;
     if (s->plan && s->plan->stream) (void)hipStreamSynchronize(s->plan->stream);
-    for (void* p : {(void*)s->win, (void*)s->head, (void*)s->acc, (void*)s->pend, (void*)s->total,
-                    (void*)s->tile, (void*)s->d_imm, (void*)s->d_taus_snap})
+    for (void* p : {(void*)s->state, (void*)s->d_imm})
         if (p) (void)hipFree(p);
     if (s->h_imm) (void)hipHostFree(s->h_imm);
     if (s->done) (void)hipEventDestroy(s->done);
