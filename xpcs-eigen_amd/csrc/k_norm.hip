@@ -5,22 +5,29 @@
 //                   integer sums of G2/IP/IF per tau (flat-field weighted sums in
 //                   FP64 when a flat field is set) and a Welford of
 //                   x_p = N G2_p / (IP_p IF_p) with 0/0 -> 0 over each of the
-//                   chunk's two pixel slices, the two merged in order.
+//                   chunk's pixel slices, merged in order.
 //   k_norm_group    per (group, tau): sums of the group's chunks in order;
 //                   g2s = c_s N sum G2 / (sum IP sum IF)            (FP64)
 //   k_norm_q        per (q, tau): mean of the non-NaN g2s of q; the chunk
 //                   Welford states merged in order (Chan et al.), giving
 //                   stderr = sqrt(1/n) sqrt(M2/n) with every pixel of q counted.
 // The reduction order is fixed, so results are deterministic.
+#include <type_traits>
+
 #include "device_util.h"
 #include "internal.h"
 
 namespace xpcs {
 
 constexpr int kNormBatch = 8;
-constexpr int kNormBlock = 256;
-constexpr int kNormSlices = 2;                        // pixel slices of a chunk (2: measured best of 1, 2, 4, 8)
-constexpr int kNormLanes = kNormBlock / kNormSlices;  // taus per pass
+constexpr int kNormLanes = 128;                       // taus per pass
+// Pixel slices of a chunk.  Plans whose chunks fill the chip: 2 (measured best
+// of 1, 2, 4, 8).  Plans of at most kNormFewChunks chunks, where a launch lasts
+// as long as one thread's walk over its slice: 8 (128 x 128, T = 30: 28 -> 13 us;
+// at 517 x 389, about 500 chunks, 87 -> 96 us).  The choice depends on the q-map alone, so a
+// stream's snapshots and a plan of the same frames slice alike.
+constexpr int kNormSlicesMany = 2, kNormSlicesFew = 8;
+constexpr int kNormFewChunks = 512;
 
 // Running state of one (chunk slice, tau): the sums and a Welford of x_p.
 struct NormAcc {
@@ -154,26 +161,26 @@ __device__ __forceinline__ void norm_merge(NormAcc& a, const NormAcc& b)
     a.n = n;
 }
 
-// Each chunk's pixels are split into kNormSlices consecutive slices, one
-// thread per (slice, tau) for each pass of up to kNormLanes taus, and the
-// slice states are merged in slice order through LDS. A workgroup takes
-// kNormBlock / (kNormSlices * lanes) chunks at once (several when the tau
-// range is narrow, as in stream snapshots). Neither the tau range nor the
+// Each chunk's pixels are split into SL consecutive slices, one thread per
+// (slice, tau) for each pass of up to kNormLanes taus, and the slice states
+// are merged in slice order through LDS. A workgroup takes as many chunks at
+// once as its threads hold (several when the tau range is narrow, as in
+// stream snapshots). Neither the tau range nor the
 // number of chunks per workgroup changes a chunk's computation, so a range of
 // taus gets the same partials as the full schedule.
-template <int MODE, bool W32>
-__global__ void __launch_bounds__(kNormBlock)
+template <int MODE, bool W32, int SL>
+__global__ void __launch_bounds__(SL * kNormLanes)
 k_norm_partial(const NormChunk* __restrict__ chunks, int32_t nchunks, const TauParam* __restrict__ taus,
                int32_t t0, int32_t t1, int32_t S, const int64_t* __restrict__ G2, const int64_t* __restrict__ IP,
                const int64_t* __restrict__ IF, const double* __restrict__ weight,
                const uint64_t* __restrict__ pix_total, int64_t hw, NormPartial* __restrict__ part)
 {
-    __shared__ __align__(16) unsigned char s_raw[kNormBlock * sizeof(NormAcc)];
+    __shared__ __align__(16) unsigned char s_raw[SL * kNormLanes * sizeof(NormAcc)];
     NormAcc* s_acc = reinterpret_cast<NormAcc*>(s_raw);
     const int nt = t1 - t0;
     const int lanes = min(nt, kNormLanes);              // taus per pass
-    const int per_chunk = kNormSlices * lanes;
-    const int cpb = max(1, kNormBlock / per_chunk);     // chunks per workgroup (the launch sizes the block to it)
+    const int per_chunk = SL * lanes;
+    const int cpb = (int)blockDim.x / per_chunk;        // chunks per workgroup
     const int cc = (int)threadIdx.x / per_chunk;
     const int r = (int)threadIdx.x % per_chunk;
     const int sl = r / lanes, lt = r % lanes;
@@ -183,8 +190,8 @@ k_norm_partial(const NormChunk* __restrict__ chunks, int32_t nchunks, const TauP
         NormChunk ch{0, 0};
         if (live) ch = chunks[c];
         const int len = ch.end - ch.begin;
-        const int pb = ch.begin + (int)((int64_t)len * sl / kNormSlices);
-        const int pe = ch.begin + (int)((int64_t)len * (sl + 1) / kNormSlices);
+        const int pb = ch.begin + (int)((int64_t)len * sl / SL);
+        const int pe = ch.begin + (int)((int64_t)len * (sl + 1) / SL);
         for (int tb = t0; tb < t1; tb += lanes) {   // uniform trip count
             const int i = tb + lt;
             const bool act = live && i < t1;
@@ -197,7 +204,7 @@ k_norm_partial(const NormChunk* __restrict__ chunks, int32_t nchunks, const TauP
             if (act && sl == 0) {
                 NormAcc a = s_acc[threadIdx.x];
 #pragma unroll
-                for (int k = 1; k < kNormSlices; k++) norm_merge<MODE>(a, s_acc[threadIdx.x + k * lanes]);
+                for (int k = 1; k < SL; k++) norm_merge<MODE>(a, s_acc[threadIdx.x + k * lanes]);
                 NormPartial o;
                 constexpr bool fpsum = MODE != kNormInt;
                 o.g2 = fpsum ? __double_as_longlong(a.wg) : a.sg;
@@ -398,20 +405,22 @@ void launch_normalize_sums(xpcs_mt_plan* p, hipStream_t s, int32_t t0, int32_t t
     const int32_t nt = t1 - t0;
     if (nt <= 0) return;
     timer_begin(p, s, "k_norm");
-    // chunks per workgroup as the kernel derives them from the tau range
-    const int cpb = std::max(1, kNormBlock / (kNormSlices * std::min(nt, kNormLanes)));
-    const int64_t nwg = (nchunks + cpb - 1) / cpb;
-    const unsigned nb = nwg < 65536 ? (unsigned)nwg : 65536u;
-    // only the threads the chunks use, whole waves (T = 88: 192 threads, not 256)
-    const int used = cpb * kNormSlices * std::min(nt, kNormLanes);
-    const int nthr = std::min(kNormBlock, (used + 63) / 64 * 64);
-    if (nchunks > 0) {
-        auto k = fp       ? k_norm_partial<kNormFp, false>
-                 : weight ? (w32 ? k_norm_partial<kNormWeighted, true> : k_norm_partial<kNormWeighted, false>)
-                 : (w32 ? k_norm_partial<kNormInt, true> : k_norm_partial<kNormInt, false>);
+    auto partial = [&](auto slices, int most) {
+        constexpr int SL = decltype(slices)::value;
+        // whole waves of the threads the chunks use (T = 88: 192, not 256)
+        const int per_chunk = SL * std::min(nt, kNormLanes);
+        const int nthr = (std::max(1, most / per_chunk) * per_chunk + 63) / 64 * 64;
+        const int cpb = nthr / per_chunk;
+        const int64_t nwg = (nchunks + cpb - 1) / cpb;
+        const unsigned nb = nwg < 65536 ? (unsigned)nwg : 65536u;
+        auto k = fp       ? k_norm_partial<kNormFp, false, SL>
+                 : weight ? (w32 ? k_norm_partial<kNormWeighted, true, SL> : k_norm_partial<kNormWeighted, false, SL>)
+                 : (w32 ? k_norm_partial<kNormInt, true, SL> : k_norm_partial<kNormInt, false, SL>);
         k<<<nb, nthr, 0, s>>>(p->d_chunks, nchunks, taus, t0, t1, S, G2, IP, IF, weight, p->d_pix_total,
                               (int64_t)h.P * S, out.part);
-    }
+    };
+    if (nchunks > kNormFewChunks) partial(std::integral_constant<int, kNormSlicesMany>{}, kNormSlicesMany * kNormLanes);
+    else if (nchunks > 0) partial(std::integral_constant<int, kNormSlicesFew>{}, 64);
     const int64_t ng = (int64_t)h.ngroups * nt;
     if (ng > 0)
         k_norm_group<<<(unsigned)ng, 64, 0, s>>>(out.part, p->d_group_chunk_first, p->d_group_size, h.ngroups,
