@@ -385,7 +385,7 @@ struct StreamLaunch {
     uint64_t* total;
 };
 void launch_stream_update(const StreamLaunch& a, hipStream_t s);
-void launch_stream_snapshot(const StreamLaunch& a, int32_t n, const LevelParam* levels, int32_t nlev,
+void launch_stream_snapshot(const StreamLaunch& a, int32_t n, const LevelParam* levels, const TauParam* taus_host,
                             const TauParam* taus_max, int32_t t0, int32_t t1, int32_t S, TauParam* taus,
                             int64_t* G2, int64_t* IP, int64_t* IF, hipStream_t s);
 void enqueue_execute(xpcs_mt_plan* p, hipStream_t s);

@@ -24,7 +24,7 @@ constexpr int kNormLanes = 128;                       // taus per pass
 // Pixel slices of a chunk.  Plans whose chunks fill the chip: 2 (measured best
 // of 1, 2, 4, 8).  Plans of at most kNormFewChunks chunks, where a launch lasts
 // as long as one thread's walk over its slice: 8 (128 x 128, T = 30: 28 -> 13 us;
-// at 517 x 389, about 500 chunks, 87 -> 96 us).  The choice depends on the q-map alone, so a
+// at 517 x 389, 512 to 1024 chunks, 87 -> 96 us).  The choice depends on the q-map alone, so a
 // stream's snapshots and a plan of the same frames slice alike.
 constexpr int kNormSlicesMany = 2, kNormSlicesFew = 8;
 constexpr int kNormFewChunks = 512;

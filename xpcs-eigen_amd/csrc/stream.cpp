@@ -301,8 +301,8 @@ extern "C" xpcs_status xpcs_mt_stream_snapshot(xpcs_mt_stream* s)
         }
     }
     for (int r = 0; r < nr; r++) {
-        launch_stream_snapshot(a, s->n, s->plan->d_levels, (int32_t)h.levels.size(), s->plan->d_taus, rng[r][0],
-                               rng[r][1], S, s->d_taus_snap, s->plan->d_G2, s->plan->d_IP, s->plan->d_IF, q);
+        launch_stream_snapshot(a, s->n, s->plan->d_levels, h.taus.data(), s->plan->d_taus, rng[r][0], rng[r][1], S,
+                               s->d_taus_snap, s->plan->d_G2, s->plan->d_IP, s->plan->d_IF, q);
         launch_normalize_with(s->plan, q, rng[r][0], rng[r][1], S, s->d_taus_snap);
     }
     HIP_TRY(hipGetLastError());
