@@ -349,7 +349,8 @@ xpcs_status xpcs_mt_set_timing_filter(xpcs_mt_plan* plan, const char* name);
 /*
  * Launch shapes of a plan (no reference counterpart: the reference's only knob
  * is the OpenMP schedule of multiTau2, src/xpcs/corr.cpp:329).  0 = automatic.
- *   tr_bucket_shift  pixels per transpose bucket = 2^shift (8..12)
+ *   tr_bucket_shift  pixels per transpose bucket = 2^shift (8..12; 0 from
+ *                    get_tuning: the automatic choice is 2^7)
  *   tr_chunk_frames  raw frames per transpose workgroup (>= 1)
  *   reg_blocks       workgroups of the register-resident row kernel (1..65535)
  *   lds_blocks       workgroups of the LDS row kernel (1..65535)

@@ -1143,7 +1143,7 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
             if (st) return st;
             p->ev_cap = p->raw_events;
         }
-        p->tshape = transpose_shape(p->nrows, p->nsel, p->tune.tr_bucket_shift, p->tune.tr_chunk_frames);
+        p->tshape = transpose_shape(p->nrows, p->nsel, p->raw_events, p->tune.tr_bucket_shift, p->tune.tr_chunk_frames);
         // the row placement holds one bucket's cursors in LDS: 4096 rows at most
         if (p->tshape.bshift > 12)
             return fail(XPCS_ERR_UNSUPPORTED,

@@ -283,7 +283,7 @@ void set_error(const char* fmt, ...);
 xpcs_status fail(xpcs_status st, const char* fmt, ...);
 
 // kernel launchers (kernels_*.hip); all asynchronous on `s`
-TransposeShape transpose_shape(int64_t P, int64_t nsel, int32_t bucket_shift, int32_t chunk_frames);
+TransposeShape transpose_shape(int64_t P, int64_t nsel, int64_t events, int32_t bucket_shift, int32_t chunk_frames);
 int64_t bucket_scan_scratch(int32_t nb, int32_t nblk);
 // with_side: also accumulate the side statistics' frame sums into d_fs (which
 // the caller has zeroed); only when side_fused(p)

@@ -991,18 +991,32 @@ int64_t bucket_scan_scratch(int32_t nb, int32_t nblk)
     return (int64_t)((nblk + kColChunks - 1) / kColChunks) * nb + nb + 1;
 }
 
-// Buckets of 2^bshift pixel rows (at least 256: k_tr_rows scans a bucket with
-// 256 threads; at most 4096 buckets: the per-chunk LDS histogram; by default
-// about 1024, which keeps each chunk's bucket segments long), cf raw frames
-// per chunk workgroup (default: at most 1024 chunks).  bucket_shift and
-// chunk_frames override the defaults when non-zero.
-TransposeShape transpose_shape(int64_t P, int64_t nsel, int32_t bucket_shift, int32_t chunk_frames)
+// Buckets of 2^bshift pixel rows (at most 4096 buckets: the per-chunk LDS
+// histogram; by default about 1024, which keeps each chunk's bucket segments
+// long), cf raw frames per chunk workgroup (default: at most 1024 chunks).
+// Buckets of more events than k_tr_rows stages (four ranges of nearly
+// kTrRowsCap) are halved, down to 128 rows, while the mean is above that:
+// 600 x 600 with 100 M events, 142k a bucket at 512 rows and 36k at 128:
+// k_tr_rows 865 -> 416 us, the row kernels, which get better sorted rows,
+// 1037 -> 951 us, k_tr_count 258 -> 219 us, against k_tr_bucket's shorter
+// segments 525 -> 725 us.  (1024 x 1024 with 41 M events, 40k a bucket:
+// halving cost 60 us in all, so there is no halving below the limit.)
+// bucket_shift and chunk_frames override the defaults when non-zero.
+constexpr int64_t kTrBucketEvents = 4 * (kTrRowsCap - 512);
+constexpr int kTrMinShift = 7;
+
+TransposeShape transpose_shape(int64_t P, int64_t nsel, int64_t events, int32_t bucket_shift, int32_t chunk_frames)
 {
     TransposeShape t;
     t.bshift = 8;
     if (bucket_shift > 8) t.bshift = bucket_shift;
-    else if (bucket_shift == 0)
-        while (((P + (int64_t(1) << t.bshift) - 1) >> t.bshift) > 1024) t.bshift++;
+    else if (bucket_shift == 0) {
+        auto buckets = [&](int shift) { return (P + (int64_t(1) << shift) - 1) >> shift; };
+        while (buckets(t.bshift) > 1024) t.bshift++;
+        while (t.bshift > kTrMinShift && buckets(t.bshift - 1) <= 4096 &&
+               events > kTrBucketEvents * buckets(t.bshift))
+            t.bshift--;
+    }
     while (((P + (int64_t(1) << t.bshift) - 1) >> t.bshift) > 4096) t.bshift++;
     t.nb = (int32_t)((P + (int64_t(1) << t.bshift) - 1) >> t.bshift);
     t.cf = nsel > 1024 ? (nsel + 1023) / 1024 : 1;
