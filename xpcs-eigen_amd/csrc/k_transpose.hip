@@ -696,16 +696,26 @@ k_tr_colsum(const uint32_t* __restrict__ hist, int32_t nb, int32_t nblk, int64_t
     part[(int64_t)blockIdx.y * nb + b] = sum;
 }
 
+// A column has at most 64 segments by default and a launch few threads, so its
+// time is the waits of one thread: 16 values are loaded at a time
+// (1000 chunks: 16.9 -> 5.6 us).
+constexpr int kColBatch = 16;
+
 __global__ void __launch_bounds__(kScanBlock)
 k_tr_colscan(int64_t* __restrict__ part, int32_t nb, int32_t nseg, int64_t* __restrict__ total)
 {
     const int32_t b = blockIdx.x * kScanBlock + threadIdx.x;
     if (b >= nb) return;
     int64_t run = 0;
-    for (int32_t r = 0; r < nseg; r++) {
-        const int64_t v = part[(int64_t)r * nb + b];
-        part[(int64_t)r * nb + b] = run;
-        run += v;
+    for (int32_t r0 = 0; r0 < nseg; r0 += kColBatch) {
+        int64_t v[kColBatch];
+#pragma unroll
+        for (int j = 0; j < kColBatch; j++) v[j] = r0 + j < nseg ? part[(int64_t)(r0 + j) * nb + b] : 0;
+#pragma unroll
+        for (int j = 0; j < kColBatch; j++) {
+            if (r0 + j < nseg) part[(int64_t)(r0 + j) * nb + b] = run;
+            run += v[j];
+        }
     }
     total[b] = run;
 }
