@@ -42,6 +42,19 @@ static xpcs_status dalloc(T** p, size_t n)
     return XPCS_OK;
 }
 
+// A workspace of at least n elements.  Each buffer has a capacity of its own,
+// 0 while it has no memory, so that neither another buffer's size nor a failed
+// allocation can stand for it.
+template <typename T>
+static xpcs_status reserve(T** p, size_t* cap, size_t n)
+{
+    if (*p && n <= *cap) return XPCS_OK;
+    *cap = 0;
+    const xpcs_status st = dalloc(p, n);
+    if (!st) *cap = n;
+    return st;
+}
+
 template <typename T>
 static xpcs_status upload(T** p, const std::vector<T>& v, hipStream_t s)
 {
@@ -502,12 +515,8 @@ xpcs_status finish_selection(xpcs_mt_plan* p, const std::vector<int64_t>& sel_of
     p->nsel = (int64_t)n;
     // offsets, lengths and output frames in one kept buffer, one copy
     const size_t bytes = std::max<size_t>(n, 1) * (sizeof(int64_t) + sizeof(uint32_t) + sizeof(int32_t));
-    if (bytes > p->sel_cap) {
-        p->sel_cap = 0;
-        const xpcs_status st = dalloc(&p->d_sel, bytes);
-        if (st) return st;
-        p->sel_cap = bytes;
-    }
+    const xpcs_status st = reserve(&p->d_sel, &p->sel_cap, bytes);
+    if (st) return st;
     p->d_sel_off = reinterpret_cast<int64_t*>(p->d_sel);
     p->d_sel_dlen = reinterpret_cast<uint32_t*>(p->d_sel_off + n);
     p->d_sel_frame = reinterpret_cast<int32_t*>(p->d_sel_dlen + n);
@@ -729,12 +738,8 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
         const size_t fb = (size_t)h.W * (size_t)h.H * 2;
         std::vector<int64_t> doff;
         if (h.darks > 0) {
-            if (fb * (size_t)h.darks > p->dark_cap) {
-                p->dark_cap = 0;
-                st = dalloc(&p->d_dark_raw, fb * (size_t)h.darks);
-                if (st) return st;
-                p->dark_cap = fb * (size_t)h.darks;
-            }
+            st = reserve(&p->d_dark_raw, &p->dark_cap, fb * (size_t)h.darks);
+            if (st) return st;
             for (int i = 0; i < h.darks; i++) {
                 doff.push_back((int64_t)(fb * (size_t)i));
                 st = h2d_staged(p->d_dark_raw + doff.back(), b + off[(size_t)i], fb, p->stream);
@@ -760,11 +765,8 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
     const size_t len = hi - lo;
     // the tail pad keeps tile loads of the last frame inside the allocation
     const size_t pad = 256;
-    if (len + pad > p->imm_cap) {
-        st = dalloc(&p->d_imm_owned, len + pad);
-        if (st) return st;
-        p->imm_cap = len + pad;
-    }
+    st = reserve(&p->d_imm_owned, &p->imm_cap, len + pad);
+    if (st) return st;
     st = h2d_staged(p->d_imm_owned, b + lo, len, p->stream);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
@@ -836,11 +838,8 @@ extern "C" xpcs_status xpcs_mt_ingest_events(xpcs_mt_plan* p, const int32_t* pix
         }
     }
     const size_t pad = 256;
-    if (bytes + pad > p->imm_cap) {
-        st = dalloc(&p->d_imm_owned, bytes + pad);
-        if (st) return st;
-        p->imm_cap = bytes + pad;
-    }
+    st = reserve(&p->d_imm_owned, &p->imm_cap, bytes + pad);
+    if (st) return st;
     st = h2d_staged(p->d_imm_owned, buf.data(), bytes, p->stream);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
@@ -941,11 +940,8 @@ extern "C" xpcs_status xpcs_mt_ingest_packed(xpcs_mt_plan* p, const void* words,
         }
     }
     const size_t len = (size_t)(hi - lo) * (size_t)wb;
-    if (len + 256 > p->imm_cap) {
-        st = dalloc(&p->d_imm_owned, len + 256);
-        if (st) return st;
-        p->imm_cap = len + 256;
-    }
+    st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
+    if (st) return st;
     st = h2d_staged(p->d_imm_owned, static_cast<const uint8_t*>(words) + (size_t)lo * (size_t)wb, len, p->stream);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
@@ -993,11 +989,8 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
     const int64_t npd = (int64_t)h.W * h.H;
     const int64_t f_lo = sel.front(), f_hi = sel.back() + 1;
     const size_t len = (size_t)(f_hi - f_lo) * (size_t)npd * 2;
-    if (len + 256 > p->imm_cap) {
-        st = dalloc(&p->d_imm_owned, len + 256);
-        if (st) return st;
-        p->imm_cap = len + 256;
-    }
+    st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
+    if (st) return st;
     if (bytes_per_value == 2) {
         st = h2d_staged(p->d_imm_owned, static_cast<const uint8_t*>(frames) + (size_t)f_lo * npd * 2, len, p->stream);
     } else {
@@ -1075,11 +1068,10 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
         }
         if (row_off[j + 1] - row_off[j] <= reg_cap() && tot > 0xFFFFFFFFull) wide = true;
     }
-    xpcs_status st = dalloc(&p->d_ev, ev.size() + kRowSlack);
+    const xpcs_status st = reserve(&p->d_ev, &p->ev_cap, ev.size() + kRowSlack);
     if (st) return st;
     if (!ev.empty())
         HIP_TRY(hipMemcpyAsync(p->d_ev, ev.data(), ev.size() * sizeof(uint64_t), hipMemcpyHostToDevice, p->stream));
-    p->ev_cap = (int64_t)ev.size();
     HIP_TRY(hipMemcpyAsync(p->d_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice, p->stream));
     p->events = off[(size_t)h.P];
     p->nscale = 1;
@@ -1128,21 +1120,14 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
         rank_lds_setup(p);
         int stride = 0;
         if (deep_level(p, &stride) < (int)h.levels.size()) {
-            const size_t need = (size_t)h.P * (size_t)stride;
-            if (need > p->deep_cap) {
-                xpcs_status st = dalloc(&p->d_deep, need);
-                if (st) return st;
-                p->deep_cap = need;
-            }
+            const xpcs_status st = reserve(&p->d_deep, &p->deep_cap, (size_t)h.P * (size_t)stride);
+            if (st) return st;
         }
     }
     if (p->mode == 1) {
-        if (!p->d_ev || p->raw_events > p->ev_cap) {
-            xpcs_status st = dalloc(&p->d_ev, (size_t)p->raw_events + kRowSlack);
-            if (!st) st = dalloc(&p->d_b1, (size_t)p->raw_events);
-            if (st) return st;
-            p->ev_cap = p->raw_events;
-        }
+        xpcs_status st = reserve(&p->d_ev, &p->ev_cap, (size_t)p->raw_events + kRowSlack);
+        if (!st) st = reserve(&p->d_b1, &p->b1_cap, (size_t)p->raw_events);
+        if (st) return st;
         p->tshape = transpose_shape(p->nrows, p->nsel, p->raw_events, p->tune.tr_bucket_shift, p->tune.tr_chunk_frames);
         // the row placement holds one bucket's cursors in LDS: 4096 rows at most
         if (p->tshape.bshift > 12)
@@ -1150,18 +1135,10 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
                         "execute: the sparse transpose takes at most 4096 x 4096 detector pixels, not %lld",
                         (long long)p->nrows);
         const int64_t nh = (int64_t)p->tshape.nb * p->tshape.nblk;
-        if (nh + 1 > p->hist_cap) {
-            xpcs_status st = dalloc(&p->d_hist, (size_t)nh);
-            if (!st) st = dalloc(&p->d_hoff, (size_t)nh + 1);
-            if (st) return st;
-            p->hist_cap = nh + 1;
-        }
-        const int64_t nbs = bucket_scan_scratch(p->tshape.nb, p->tshape.nblk);
-        if (nbs > p->bsum_cap) {
-            xpcs_status st = dalloc(&p->d_bsum, (size_t)nbs);
-            if (st) return st;
-            p->bsum_cap = nbs;
-        }
+        st = reserve(&p->d_hist, &p->hist_cap, (size_t)nh);
+        if (!st) st = reserve(&p->d_hoff, &p->hoff_cap, (size_t)nh + 1);
+        if (!st) st = reserve(&p->d_bsum, &p->bsum_cap, (size_t)bucket_scan_scratch(p->tshape.nb, p->tshape.nblk));
+        if (st) return st;
     } else if (dense_stream) {
         if (!p->d_wave_flags) {
             // one flag per wave of the dense kernels' grids (whole workgroups of 256)
@@ -1169,19 +1146,12 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
             if (st) return st;
         }
         const size_t need = dense_series_elems(p);
-        if (need > p->series_cap) {
-            xpcs_status st = dalloc(&p->d_series_a, need);
-            if (!st) st = dalloc(&p->d_series_b, need);
-            if (st) return st;
-            p->series_cap = need;
-        }
+        xpcs_status st = reserve(&p->d_series_a, &p->series_a_cap, need);
+        if (!st) st = reserve(&p->d_series_b, &p->series_b_cap, need);
+        if (st) return st;
     } else if (p->mode == 2) {
-        const size_t need = (size_t)h.P * (size_t)h.F;
-        if (need > p->rows_cap) {
-            xpcs_status st = dalloc(&p->d_rows, need);
-            if (st) return st;
-            p->rows_cap = need;
-        }
+        const xpcs_status st = reserve(&p->d_rows, &p->rows_cap, (size_t)h.P * (size_t)h.F);
+        if (st) return st;
     }
     return XPCS_OK;
 }

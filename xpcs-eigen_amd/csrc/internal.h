@@ -180,15 +180,16 @@ struct xpcs_mt_plan {
     size_t dark_cap = 0;
 
     // events (pixel-major CSR over compact pixels)
-    int64_t ev_cap = 0;
+    size_t ev_cap = 0;                   // of d_ev, kRowSlack included
     uint64_t* d_ev = nullptr;            // (frame << 32) | count
     int64_t* d_off = nullptr;            // [P+1]
     uint64_t* d_b1 = nullptr;            // bucketed events (transpose stage)
+    size_t b1_cap = 0;
     uint32_t* d_hist = nullptr;          // [nblk][nb] events per (chunk, bucket)
     int64_t* d_hoff = nullptr;           // [nblk][nb] segment starts, then the total
-    int64_t hist_cap = 0;
+    size_t hist_cap = 0, hoff_cap = 0;
     int64_t* d_bsum = nullptr;           // bucket scan scratch
-    int64_t bsum_cap = 0;
+    size_t bsum_cap = 0;
     xpcs::TransposeShape tshape;
     int64_t events = 0;                  // known after execute (host copy)
     // dense rows (fallback path)
@@ -209,7 +210,7 @@ struct xpcs_mt_plan {
     // dense streaming path: coarsened series between passes, boundary events
     uint32_t* d_series_a = nullptr;
     uint32_t* d_series_b = nullptr;
-    size_t series_cap = 0;
+    size_t series_a_cap = 0, series_b_cap = 0;
     int4* d_bnd = nullptr;               // (frame boundary, op, tau slot, 0), sorted
     int32_t nbnd = 0;
     int32_t* d_cap = nullptr;            // the distinct boundaries B_j and an entry beyond every frame
