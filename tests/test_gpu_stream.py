@@ -140,6 +140,22 @@ def test_stream_errors(xmt):
         s.g2()
 
 
+@pytest.mark.parametrize("read", ["g2", "sums"])
+def test_error_pushed_after_the_snapshot(xmt, read):
+    """A bad pixel index is reported by the next read, snapshot or not."""
+    c = cases.sparse_case(W=16, H=16, F=60, dpl=4, mu=0.3, tau_c=5.0, seed=7)
+    s = xmt.Stream(16, 16, 60, 4, c["dq"], c["sq"])
+    s.push_imm(synth.imm_bytes_sparse(c["counts"][:50], 16, 16))
+    s.snapshot()
+    getattr(s, read)()
+    bad = bytearray(synth.imm_bytes_sparse(c["counts"][50:52], 16, 16))
+    bad[1024:1028] = int(16 * 16 + 5).to_bytes(4, "little")
+    s.push_imm(bytes(bad))
+    with pytest.raises(xmt.XpcsError, match="RANGE"):
+        getattr(s, read)()
+    s.close()
+
+
 def test_service_mix_equals_alone(xmt):
     import serve
     streams = []

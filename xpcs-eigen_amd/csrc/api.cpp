@@ -281,7 +281,6 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
     }
     mem.buffer(&p->d_long_list, (size_t)h.P);
     mem.buffer(&p->d_mid_list, (size_t)h.P);
-    mem.buffer(&p->d_counters, 8);
     {
         // level-0 prefix boundaries of the dense streaming path
         std::vector<int4> bnd;
@@ -331,9 +330,10 @@ extern "C" xpcs_status xpcs_mt_plan_create(const xpcs_mt_desc* desc, xpcs_mt_pla
         if (p->fsnorm) p->long_blocks = (int)std::min<size_t>(8192, std::max<size_t>(1, 4 * budget / per));
     }
     TRY(mem.commit(&p->d_arena, s));
+    p->d_counters = reinterpret_cast<RunStatus*>(p->d_stat)->counters;
     p->d_g2 = reinterpret_cast<double*>(p->d_stat + sizeof(RunStatus) / sizeof(int64_t));
     p->d_se = p->d_g2 + QT;
-    if (hipMemsetAsync(p->d_counters, 0, 32, s) != hipSuccess ||
+    if (hipMemsetAsync(p->d_stat, 0, sizeof(RunStatus), s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         xpcs_mt_plan_destroy(p);
         return fail(XPCS_ERR_HIP, "plan_create: initialisation failed");
@@ -1166,7 +1166,7 @@ void enqueue_execute(xpcs_mt_plan* p, hipStream_t s)
     // bytes), recorded with the launches that write them, so the readers follow
     // the last multi-tau run whatever ran on the plan since
     p->ipif32 = !p->fsnorm && p->tune.sums64 == 0;
-    launch_fill_u32(p->d_counters, 8, s);
+    launch_fill_u32(p->d_counters, kCounters, s);
     if (p->d_fs) launch_fill_u64(reinterpret_cast<uint64_t*>(p->d_fs), (size_t)h.F * h.ns, s);
     if (p->fsnorm && p->mode == 2 && dense_stream_ok(p)) {
         // normalize_by_framesum on dense frames: frame sums from the raw
@@ -1229,7 +1229,7 @@ static xpcs_status sync_and_check(xpcs_mt_plan* p, double* g2 = nullptr, double*
     collect_timers(p);
     RunStatus r;
     std::memcpy(&r, p->h_result.data(), sizeof(r));
-    if (r.errors & 1u) return fail(XPCS_ERR_RANGE, "execute: an IMM pixel index lies outside the detector");
+    if (r.counters[1] & 1u) return fail(XPCS_ERR_RANGE, "execute: an IMM pixel index lies outside the detector");
     if (p->mode == 1) p->events = r.events;
     const size_t half = (size_t)p->h.nq * p->h.T * sizeof(double);
     if (g2) std::memcpy(g2, p->h_result.data() + sizeof(r), half);

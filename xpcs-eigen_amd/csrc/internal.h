@@ -82,11 +82,14 @@ struct TransposeShape {
     int32_t nblk = 1;     // chunks
 };
 
-// What a run leaves beside its results (written by the last normalisation kernel).
+constexpr int kCounters = 8;   // d_counters
+
+// What a run leaves beside its results, which follow it in memory, so that one
+// copy reads both.  The counters are the ones the kernels set: an error shows
+// in the next read whether or not a normalisation ran after it.
 struct RunStatus {
-    int64_t events;      // level-0 events of the transposed rows
-    uint32_t errors;     // error flags of the transpose
-    uint32_t pad;
+    uint32_t counters[kCounters];
+    int64_t events;      // level-0 events of the transposed rows (written by the last normalisation kernel)
 };
 static_assert(sizeof(RunStatus) % sizeof(int64_t) == 0, "the results follow it");
 
@@ -229,7 +232,7 @@ struct xpcs_mt_plan {
     int32_t* d_long_list = nullptr;      // [P]
     int32_t* d_mid_list = nullptr;       // [P] rows of 65..CAP events
     int32_t* d_wide_list = nullptr;      // [P] rows of at most 1024 events whose total passes 65535
-    uint32_t* d_counters = nullptr;      // [0] rows over 1024 events, [1] error flags, [2] rows of 65..128,
+    uint32_t* d_counters = nullptr;      // in d_stat: [0] rows over 1024 events, [1] error flags, [2] rows of 65..128,
                                          // [3] dense exact-redo pixels, [4] rows of 129..512, [5] 513..1024,
                                          // [6] rows in d_wide_list
     uint32_t* d_deep = nullptr;          // [P][deep stride] level series handed to the one-lane-per-pixel kernel
@@ -324,8 +327,7 @@ struct NormOut {
     double* g2;
     double* se;
     RunStatus* stat;            // NULL: not written
-    const uint32_t* counters;   // what it is taken from
-    const int64_t* events;
+    const int64_t* events;      // its event count
 };
 NormOut plan_norm_out(xpcs_mt_plan* p);
 void launch_normalize_sums(xpcs_mt_plan* p, hipStream_t s, int32_t t0, int32_t t1, int32_t S,

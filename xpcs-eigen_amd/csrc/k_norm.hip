@@ -297,15 +297,11 @@ __global__ void __launch_bounds__(64)
 k_norm_q(const NormPartial* __restrict__ part, const double* __restrict__ g2s,
          const int32_t* __restrict__ q_first_group, const int32_t* __restrict__ q_chunk_first,
          int32_t nq, int32_t t0, int32_t t1, int32_t S, double* __restrict__ g2, double* __restrict__ se,
-         RunStatus* __restrict__ stat, const uint32_t* __restrict__ counters, const int64_t* __restrict__ events)
+         RunStatus* __restrict__ stat, const int64_t* __restrict__ events)
 {
     const int64_t k = blockIdx.x;
     const int nt = t1 - t0;
-    if (stat && k == 0 && threadIdx.x == 0) {
-        stat->events = *events;
-        stat->errors = counters[1];
-        stat->pad = 0u;
-    }
+    if (stat && k == 0 && threadIdx.x == 0) stat->events = *events;
     if (k >= (int64_t)nq * nt) return;
     const int q = (int)(k / nt);    // 0-based
     const int i = t0 + (int)(k % nt);
@@ -428,13 +424,13 @@ void launch_normalize_sums(xpcs_mt_plan* p, hipStream_t s, int32_t t0, int32_t t
     const int64_t nqt = (int64_t)h.nq * nt;
     if (nqt > 0)
         k_norm_q<<<(unsigned)nqt, 64, 0, s>>>(out.part, out.g2s, p->d_q_first_group, p->d_q_chunk_first,
-                                              h.nq, t0, t1, S, out.g2, out.se, out.stat, out.counters, out.events);
+                                              h.nq, t0, t1, S, out.g2, out.se, out.stat, out.events);
     timer_end(p, s);
 }
 
 NormOut plan_norm_out(xpcs_mt_plan* p)
 {
-    return NormOut{p->d_part, p->d_g2s, p->d_g2, p->d_se, reinterpret_cast<RunStatus*>(p->d_stat), p->d_counters,
+    return NormOut{p->d_part, p->d_g2s, p->d_g2, p->d_se, reinterpret_cast<RunStatus*>(p->d_stat),
                    p->d_off + p->nrows};
 }
 

@@ -159,7 +159,7 @@ extern "C" xpcs_status xpcs_mt_stream_open(const xpcs_mt_desc* desc, int32_t max
     hipStream_t q = s->plan->stream;
     if (!st) {
         launch_fill_u32(s->state, words, q);
-        launch_fill_u32(s->plan->d_counters, 8, q);
+        launch_fill_u32(s->plan->d_counters, kCounters, q);
         if (hipEventCreateWithFlags(&s->done, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&s->copied, hipEventDisableTiming) != hipSuccess ||
             hipGetLastError() != hipSuccess || hipStreamSynchronize(q) != hipSuccess)
@@ -326,7 +326,8 @@ extern "C" xpcs_status xpcs_mt_stream_poll(xpcs_mt_stream* s, int32_t* frames_do
     return XPCS_OK;
 }
 
-// Waits for the newest snapshot; its errors, and g2 / stderr when asked for.
+// Waits for the newest snapshot and whatever was pushed since; the errors so
+// far, and the snapshot's g2 / stderr when asked for.
 static xpcs_status stream_wait(xpcs_mt_stream* s, double* g2 = nullptr, double* se = nullptr)
 {
     if (s->snap_T <= 0) return fail(XPCS_ERR_STATE, "stream: no snapshot taken");
@@ -339,7 +340,7 @@ static xpcs_status stream_wait(xpcs_mt_stream* s, double* g2 = nullptr, double* 
     s->done_n = s->snap_n;
     RunStatus r;
     std::memcpy(&r, p->h_result.data(), sizeof(r));
-    if (r.errors & 1u) return fail(XPCS_ERR_RANGE, "stream: an IMM pixel index lies outside the detector");
+    if (r.counters[1] & 1u) return fail(XPCS_ERR_RANGE, "stream: an IMM pixel index lies outside the detector");
     const size_t n = (size_t)s->snap_T * p->h.nq * sizeof(double);
     if (g2) std::memcpy(g2, p->h_result.data() + sizeof(r), n);
     if (se) std::memcpy(se, p->h_result.data() + sizeof(r) + half, n);
