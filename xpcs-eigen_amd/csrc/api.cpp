@@ -350,7 +350,7 @@ extern "C" xpcs_status xpcs_mt_plan_destroy(xpcs_mt_plan* p)
     dfree(p->d_arena); dfree(p->d_sel);
     dfree(p->d_imm_owned); dfree(p->d_dark_sum); dfree(p->d_dark_avg); dfree(p->d_dark_std); dfree(p->d_dark_isum); dfree(p->d_dark_raw);
     dfree(p->d_thr); dfree(p->d_ev); dfree(p->d_b1); dfree(p->d_hist); dfree(p->d_hoff); dfree(p->d_bsum);
-    dfree(p->d_rows); dfree(p->d_wide_list); dfree(p->d_wave_flags); dfree(p->d_scratch); dfree(p->d_deep); dfree(p->d_series_a);
+    dfree(p->d_rows); dfree(p->d_wide_list); dfree(p->d_wide_flags); dfree(p->d_wave_flags); dfree(p->d_scratch); dfree(p->d_deep); dfree(p->d_series_a);
     dfree(p->d_series_b);
     for (auto& t : p->pending) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     for (auto e : p->event_pool) (void)hipEventDestroy(e);
@@ -1055,18 +1055,22 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
         return fail(XPCS_ERR_NOMEM, "ingest_rows: %lld events do not fit host memory", (long long)off[(size_t)h.P]);
     }
     bool wide = false;   // a row short enough for the register kernels totals 2^32 or more
+    int64_t big_rows = 0;
     for (int c = 0; c < h.P; c++) {
         const int64_t j = h.order[(size_t)c];
         int64_t o = off[(size_t)c];
         uint64_t tot = 0;
+        uint32_t most = 0;
         for (int64_t e = row_off[j]; e < row_off[j + 1]; e++) {
             if (frame[e] < 0 || frame[e] >= h.F)
                 return fail(XPCS_ERR_RANGE, "ingest_rows: frame %d of pixel %lld outside [0, %d)", frame[e],
                             (long long)j, h.F);
             ev[(size_t)o++] = ((uint64_t)(uint32_t)frame[e] << 32) | count[e];
             tot += count[e];
+            most = std::max(most, count[e]);
         }
         if (row_off[j + 1] - row_off[j] <= reg_cap() && tot > 0xFFFFFFFFull) wide = true;
+        if (row_off[j + 1] - row_off[j] <= kSparseCap && most > 65535u) big_rows++;
     }
     const xpcs_status st = reserve(&p->d_ev, &p->ev_cap, ev.size() + kRowSlack);
     if (st) return st;
@@ -1078,6 +1082,7 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
     p->fmt = kFmtImm;
     p->mode = 3;
     p->wide_rows = wide;
+    p->big_rows = big_rows;
     p->nrows = h.P;
     p->d_rowmap = nullptr;
     p->executed = false;
@@ -1112,10 +1117,9 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
         if (st) return st;
     }
     if ((p->mode == 1 || p->mode == 3) && rows_supported(p)) {
-        if (!p->d_wide_list) {
-            xpcs_status st = dalloc(&p->d_wide_list, (size_t)h.P);
-            if (st) return st;
-        }
+        xpcs_status st = reserve(&p->d_wide_flags, &p->wide_flags_cap, rows_wide_flags(p));
+        if (!st && rows_with_big_counts(p)) st = reserve(&p->d_wide_list, &p->wide_list_cap, (size_t)p->big_rows);
+        if (st) return st;
     } else if (p->mode == 1 || p->mode == 3) {
         rank_lds_setup(p);
         int stride = 0;

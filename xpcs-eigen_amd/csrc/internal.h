@@ -231,10 +231,13 @@ struct xpcs_mt_plan {
     // long pixels
     int32_t* d_long_list = nullptr;      // [P]
     int32_t* d_mid_list = nullptr;       // [P] rows of 65..CAP events
-    int32_t* d_wide_list = nullptr;      // [P] rows of at most 1024 events whose total passes 65535
+    int32_t* d_wide_list = nullptr;      // rows of at most 1024 events with a count above 65535
+    size_t wide_list_cap = 0;
+    uint8_t* d_wide_flags = nullptr;     // rows of at most 1024 events whose total passes 65535 (k_rows.hip)
+    size_t wide_flags_cap = 0;
     uint32_t* d_counters = nullptr;      // in d_stat: [0] rows over 1024 events, [1] error flags, [2] rows of 65..128,
                                          // [3] dense exact-redo pixels, [4] rows of 129..512, [5] 513..1024,
-                                         // [6] rows in d_wide_list
+                                         // [6] rows in d_wide_list, [7] some row is flagged in d_wide_flags
     uint32_t* d_deep = nullptr;          // [P][deep stride] level series handed to the one-lane-per-pixel kernel
     size_t deep_cap = 0;
     uint64_t* d_scratch = nullptr;
@@ -247,6 +250,7 @@ struct xpcs_mt_plan {
     int64_t* d_IF = nullptr;             //   (low words [P*T], high words of pixels with totals >= 2^32 after them)
     bool ipif32 = false;                 // integer sums of the batch path (set by enqueue_execute)
     bool wide_rows = false;              // ingest_rows: a row of <= 128 events totals 2^32 or more
+    int64_t big_rows = 0;                // ingest_rows: rows of <= 1024 events with a count above 65535
     uint64_t* d_pix_total = nullptr;     // [P] sum of level-0 values
     xpcs::NormPartial* d_part = nullptr; // [nchunks][T]
     double* d_g2s = nullptr;             // [ngroups][T]
@@ -297,8 +301,10 @@ bool side_fused(const xpcs_mt_plan* p);
 EvFormat ev_format(const xpcs_mt_plan* p);
 void launch_mt_sparse(xpcs_mt_plan* p, hipStream_t s);
 // k_rows.hip: rows of at most 1024 events, a group of lanes per row; rows
-// whose total passes 65535 are left in d_wide_list
+// with a count above 65535 are left in d_wide_list
 bool rows_supported(const xpcs_mt_plan* p);
+bool rows_with_big_counts(const xpcs_mt_plan* p);
+size_t rows_wide_flags(const xpcs_mt_plan* p);   // bytes of d_wide_flags
 int rows_series_level(const xpcs_mt_plan* p, int N);
 void launch_mt_rows(xpcs_mt_plan* p, hipStream_t s);
 // first level of the one-lane-per-pixel kernel of the sparse path (the level

@@ -9,9 +9,10 @@
 //   IF = sum_{tau'<=t<lf_L} x_L[t] = S0(2^L lf_L) - S0(2^L tau'),
 // where S0(b) is the sum of the level-0 counts of frames < b.
 //
-// Rows of counts at 4 or 8 delays per level go through k_mt_rows (k_rows.hip)
-// unless the row total passes 65535 or the plan's frames its 16-bit keys; the
-// kernels here take the rest, and the FP64 frame-weighted values.
+// Rows of counts at 4 or 8 delays per level go through k_mt_rows and
+// k_mt_rows_wide (k_rows.hip) unless the plan's frames pass their 16-bit keys
+// or (pixel-major rows only) many rows hold counts above 65535; the kernels
+// here take the rest, and the FP64 frame-weighted values.
 //
 // k_mt_reg / k_mt_reg2: one wavefront per row of at most 64 / 128 events held
 // in registers (one / two per lane).  The row is sorted (odd-even passes, a
@@ -1809,9 +1810,10 @@ static void launch_rows(xpcs_mt_plan* p, hipStream_t s, const char* t_reg, const
         const int nl = (int)h.levels.size();
         const int64_t hwords = (int64_t)h.P * h.T;
         timer_begin(p, s, t_lds);
-        k_mt_sparse<kSparseCapMid, kSparseMidWaves, V><<<256, kWave * kSparseMidWaves, 0, s>>>(
-            p->d_ev, p->d_off, p->d_wide_list, 1, p->d_counters + 6, p->d_taus, h.T, p->d_levels, nl, h.F, p->d_G2,
-            p->d_IP, p->d_IF, p->d_pix_total, p->d_rowmap, fw, nl, p->d_deep, 0, p->ipif32, hwords);
+        if (rows_with_big_counts(p))
+            k_mt_sparse<kSparseCapMid, kSparseMidWaves, V><<<256, kWave * kSparseMidWaves, 0, s>>>(
+                p->d_ev, p->d_off, p->d_wide_list, 1, p->d_counters + 6, p->d_taus, h.T, p->d_levels, nl, h.F, p->d_G2,
+                p->d_IP, p->d_IF, p->d_pix_total, p->d_rowmap, fw, nl, p->d_deep, 0, p->ipif32, hwords);
         k_mt_sparse<kSparseCapLong, kSparseLongWaves, V><<<std::max(1, lds_blocks(p) / 4), kWave * kSparseLongWaves, 0, s>>>(
             p->d_ev, p->d_off, p->d_long_list + (h.P - 1), -1, p->d_counters, p->d_taus, h.T, p->d_levels, nl, h.F,
             p->d_G2, p->d_IP, p->d_IF, p->d_pix_total, p->d_rowmap, fw, nl, p->d_deep, 0, p->ipif32, hwords);
