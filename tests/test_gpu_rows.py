@@ -1,7 +1,9 @@
 """Row kernels (a group of lanes per pixel row): sums bit-equal to the oracle's
-at the edges of the row classes, of the row total that fits 16 bits, of the
-frame count the 16-bit keys take, with repeated frames and with frames left
-over at every level."""
+at the edges of the row classes, with repeated frames, with frames left over
+at every level and with long frame counts.  Many of the rows hold counts above
+65535, so the kernels of k_multitau.hip take them all; the same lengths and
+orders on the row kernels, the totals that fit their 16 bits and the frame
+counts that fit their keys are in test_gpu_wide_rows.py."""
 import numpy as np
 import pytest
 

@@ -1,7 +1,7 @@
-"""Rows whose counts total more than 65535, through the row kernels' wide form:
-sums bit-equal to the oracle's at the edges of the length classes and of the
-totals, mixed with narrow rows at every density, and rows with counts that do
-not fit 16 bits."""
+"""Row kernels with totals on both sides of the 65535 that 16 bits hold: sums
+bit-equal to the oracle's at the edges of the length classes, of the totals and
+of the frame counts, narrow and wide rows mixed at every density, and rows with
+counts that do not fit 16 bits."""
 import numpy as np
 import pytest
 
@@ -12,14 +12,20 @@ pytestmark = pytest.mark.gpu
 EDGES = [0, 1, 2, 7, 8, 9, 31, 63, 64, 65, 66, 127, 128, 129, 130, 500, 512, 513, 514, 1023, 1024, 1025, 1300]
 
 
-def check_rows(xmt, orc, W, H, F, dpl, frames, counts, row_kernels):
+def check_rows(xmt, orc, W, H, F, dpl, frames, counts, row_kernels, deep=0):
     """Sums of pixel-major rows against the oracle's; row_kernels: the plan takes k_mt_rows."""
     dq, sq = synth.annular_qmaps(W, H, 4, 2)
     lens = np.array([len(f) for f in frames])
     plan = xmt.Plan(W, H, F, dpl, dq, sq)
     plan.ingest_rows(np.concatenate([[0], np.cumsum(lens)]).astype(np.int64),
                      np.concatenate(frames).astype(np.int32), np.concatenate(counts).astype(np.uint32))
-    assert (plan.get_tuning()["deep_frames"] == 0) == row_kernels
+    plan.set_tuning(deep_frames=deep)
+    # the path taken: the row kernels' series has the level's frames, the other
+    # kernels' whole 16 bytes of them, by default from 96 frames on
+    info = plan.info()
+    lf = F >> info.deep_level
+    assert info.deep_stride == (lf if row_kernels else (lf + 3) & ~3)
+    assert plan.get_tuning()["deep_frames"] == (deep if deep else 0 if row_kernels else 96)
     plan.execute()
     g, a, b = plan.sums()
     total = plan.side()["pixel_sum"]
@@ -67,6 +73,35 @@ def test_wide_rows(xmt, orc, dpl, F, wide):
     rng = np.random.default_rng([dpl, F, int(100 * wide)])
     print(f"wide rows dpl={dpl} F={F} wide={wide}", flush=True)
     check_rows(xmt, orc, 20, 17, F, dpl, *draw_rows(rng, 340, F, wide), True)
+
+
+@pytest.mark.parametrize("dpl,F,deep,row_kernels", [
+    (4, 63231, 0, True), (4, 63232, 0, False), (8, 61183, 0, True), (8, 61184, 0, False),
+    (8, 65535 - 17 * 512, 96, True), (8, 65536 - 17 * 512, 96, False),
+    (4, 65535 - 9 * 2048, 16, True), (4, 65536 - 9 * 2048, 16, False),
+])
+def test_frame_limit(xmt, orc, dpl, F, deep, row_kernels):
+    """The largest frame count whose keys leave the padding key out of reach,
+    and the next one, which the other kernels take; rows with events in the
+    last frames among them."""
+    rng = np.random.default_rng(F)
+    print(f"frame limit dpl={dpl} F={F} deep_frames={deep}", flush=True)
+    check_rows(xmt, orc, 20, 17, F, dpl, *draw_rows(rng, 340, F, 0.3), row_kernels, deep)
+
+
+@pytest.mark.parametrize("order", ["sorted", "local", "shuffled"])
+@pytest.mark.parametrize("dpl,F", [(4, 1023), (8, 10007)])
+def test_narrow_rows_in_any_order(xmt, orc, dpl, F, order):
+    rng = np.random.default_rng([dpl, F, len(order)])
+    frames, counts = draw_rows(rng, 340, F, 0.0)
+    for j, f in enumerate(frames):
+        if order != "shuffled":
+            f.sort()
+        if order == "local":
+            for a in range(0, len(f), 6):
+                f[a:a + 6] = rng.permutation(f[a:a + 6])
+    print(f"rows dpl={dpl} F={F} order={order}", flush=True)
+    check_rows(xmt, orc, 20, 17, F, dpl, frames, counts, True)
 
 
 @pytest.mark.parametrize("big", [1, 10, 11])
