@@ -468,7 +468,7 @@ xpcs_status select_frames(const HostTables& h, int64_t n_raw, bool compressed, i
     return XPCS_OK;
 }
 
-xpcs_status h2d_staged(uint8_t* dst, const uint8_t* src, size_t len, hipStream_t s);
+xpcs_status h2d_staged(xpcs_mt_plan* p, uint8_t* dst, const uint8_t* src, size_t len);
 
 // Work of earlier calls may still read the buffers an ingest overwrites.  On the
 // plan's own stream the copies queue up behind it; work that went to another
@@ -533,46 +533,43 @@ xpcs_status finish_selection(xpcs_mt_plan* p, const std::vector<int64_t>& sel_of
     return XPCS_OK;
 }
 
-// Host bytes to device memory through two pinned staging buffers: while the
-// DMA engine drains one, host threads fill the other (pageable memory cannot
-// be handed to the DMA engine directly, and one thread's memcpy is slower than
-// the PCIe link).  The buffers are allocated once per process and shared by
-// all plans (one staged copy at a time).  Returns when every piece has been
-// copied; the caller's buffer is not read afterwards.
+// Two pinned buffers and the events of the last copy through each.  A device
+// has one pool, made on first use, which lives until the process ends and is
+// shared by the device's plans (one staged copy at a time).
 struct StagePool {
     std::mutex mu;
     uint8_t* buf[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};
-    size_t bytes = 0;
 };
 
-constexpr size_t kStage = size_t(32) << 20;
+constexpr size_t kStageUpload = size_t(32) << 20;
+constexpr size_t kStageRead = size_t(8) << 20;
 
-// The pool of the current device (lives until the process ends).
-StagePool& stage_pool()
+// The pool of the plan's device, whichever device is current.
+StagePool& stage_pool(const xpcs_mt_plan* p)
 {
-    static StagePool pools[16];
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    return pools[dev & 15];
+    static StagePool pools[64];   // eight GPUs of eight partitions
+    return pools[p->device & 63];
 }
 
-// The pool's buffers and events, made on first use (sp.mu held).
-xpcs_status stage_ready(StagePool& sp)
+// The pool's buffers of `bytes` and its events, made on first use (sp.mu held).
+xpcs_status stage_ready(StagePool& sp, int device, size_t bytes)
 {
     if (sp.buf[0]) return XPCS_OK;
-    for (int i = 0; i < 2; i++) {
-        if (hipHostMalloc(reinterpret_cast<void**>(&sp.buf[i]), kStage, hipHostMallocDefault) != hipSuccess ||
-            hipEventCreateWithFlags(&sp.done[i], hipEventDisableTiming) != hipSuccess) {
-            for (int j = 0; j <= i; j++) {
-                if (sp.buf[j]) (void)hipHostFree(sp.buf[j]);
-                sp.buf[j] = nullptr;
-            }
-            return fail(XPCS_ERR_NOMEM, "pinned staging of %zu bytes failed", kStage);
-        }
+    int current = device;
+    (void)hipGetDevice(&current);
+    if (current != device) (void)hipSetDevice(device);   // an event belongs to the device it is made on
+    bool ok = true;
+    for (int i = 0; i < 2; i++)
+        ok = ok && hipHostMalloc(reinterpret_cast<void**>(&sp.buf[i]), bytes, hipHostMallocDefault) == hipSuccess &&
+             (sp.done[i] || hipEventCreateWithFlags(&sp.done[i], hipEventDisableTiming) == hipSuccess);
+    if (current != device) (void)hipSetDevice(current);
+    if (ok) return XPCS_OK;
+    for (auto& b : sp.buf) {
+        if (b) (void)hipHostFree(b);
+        b = nullptr;
     }
-    sp.bytes = kStage;
-    return XPCS_OK;
+    return fail(XPCS_ERR_NOMEM, "pinned staging of %zu bytes failed", bytes);
 }
 
 // memcpy over several threads (a thread that cannot be started leaves its part
@@ -595,24 +592,29 @@ void parallel_copy(uint8_t* dst, const uint8_t* src, size_t n)
         if (th.joinable()) th.join();
 }
 
-xpcs_status h2d_staged(uint8_t* dst, const uint8_t* src, size_t len, hipStream_t s)
+// Host bytes to device memory through two pinned staging buffers: while the
+// DMA engine drains one, host threads fill the other (pageable memory cannot
+// be handed to the DMA engine directly, and one thread's memcpy is slower than
+// the PCIe link).  One upload per device at a time.  Returns when every piece
+// has been copied; the caller's buffer is not read afterwards.
+xpcs_status h2d_staged(xpcs_mt_plan* p, uint8_t* dst, const uint8_t* src, size_t len)
 {
     if (len == 0) return XPCS_OK;
-    StagePool& sp = stage_pool();
+    StagePool& sp = stage_pool(p);
     std::lock_guard<std::mutex> lk(sp.mu);
-    xpcs_status st = stage_ready(sp);
+    xpcs_status st = stage_ready(sp, p->device, kStageUpload);
     if (st) return st;
     int b = 0;
     bool issued[2] = {false, false};
-    for (size_t off = 0; off < len && !st; off += sp.bytes, b ^= 1) {
-        const size_t n = std::min(sp.bytes, len - off);
+    for (size_t off = 0; off < len && !st; off += kStageUpload, b ^= 1) {
+        const size_t n = std::min(kStageUpload, len - off);
         if (issued[b] && hipEventSynchronize(sp.done[b]) != hipSuccess) {
             st = fail(XPCS_ERR_HIP, "ingest: staging copy failed");
             break;
         }
         parallel_copy(sp.buf[b], src + off, n);   // into the pinned buffer
-        if (hipMemcpyAsync(dst + off, sp.buf[b], n, hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipEventRecord(sp.done[b], s) != hipSuccess)
+        if (hipMemcpyAsync(dst + off, sp.buf[b], n, hipMemcpyHostToDevice, p->stream) != hipSuccess ||
+            hipEventRecord(sp.done[b], p->stream) != hipSuccess)
             st = fail(XPCS_ERR_HIP, "ingest: host-to-device copy failed");
         issued[b] = true;
     }
@@ -662,28 +664,29 @@ void dense_tiling(xpcs_mt_plan* p, const std::vector<int64_t>& so, const uint8_t
 
 namespace xpcs {
 
-// Device results to pageable host memory, after the work queued on s.  Large
-// ones come through the pinned buffers a piece at a time, one piece on the
-// link while threads copy the other out (a plain copy ran at 13 GB/s, most of
-// it first-touch page faults of the caller's array on one thread).
-xpcs_status d2h_staged(void* dst, const void* src, size_t len, hipStream_t s)
+// Device results to pageable host memory, after the work queued on the plan's
+// stream.  Large ones come through the pinned buffers a piece at a time, one
+// piece on the link while threads copy the other out (a plain copy ran at 13
+// GB/s, most of it first-touch page faults of the caller's array on one
+// thread).
+xpcs_status d2h_staged(xpcs_mt_plan* p, void* dst, const void* src, size_t len)
 {
-    constexpr size_t kPiece = size_t(8) << 20;
     if (len == 0) return XPCS_OK;
+    hipStream_t s = p->stream;
     if (len < (size_t(2) << 20)) {
         HIP_TRY(hipMemcpyAsync(dst, src, len, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         return XPCS_OK;
     }
-    StagePool& sp = stage_pool();
+    StagePool& sp = stage_pool(p);
     std::lock_guard<std::mutex> lk(sp.mu);
-    xpcs_status st = stage_ready(sp);
+    xpcs_status st = stage_ready(sp, p->device, kStageUpload);
     if (st) return st;
     uint8_t* d = static_cast<uint8_t*>(dst);
     const uint8_t* q = static_cast<const uint8_t*>(src);
-    const size_t pieces = (len + kPiece - 1) / kPiece;
+    const size_t pieces = (len + kStageRead - 1) / kStageRead;
     auto issue = [&](size_t k) {
-        const size_t off = k * kPiece, n = std::min(kPiece, len - off);
+        const size_t off = k * kStageRead, n = std::min(kStageRead, len - off);
         if (hipMemcpyAsync(sp.buf[k & 1], q + off, n, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipEventRecord(sp.done[k & 1], s) != hipSuccess)
             st = fail(XPCS_ERR_HIP, "read: device-to-host copy failed");
@@ -692,7 +695,7 @@ xpcs_status d2h_staged(void* dst, const void* src, size_t len, hipStream_t s)
     for (size_t k = 0; k < pieces && !st; k++) {
         if (k + 1 < pieces) issue(k + 1);
         if (hipEventSynchronize(sp.done[k & 1]) != hipSuccess) st = fail(XPCS_ERR_HIP, "read: device-to-host copy failed");
-        if (!st) parallel_copy(d + k * kPiece, sp.buf[k & 1], std::min(kPiece, len - k * kPiece));
+        if (!st) parallel_copy(d + k * kStageRead, sp.buf[k & 1], std::min(kStageRead, len - k * kStageRead));
     }
     if (st) (void)hipStreamSynchronize(s);   // nothing may still write the pool
     return st;
@@ -742,7 +745,7 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
             if (st) return st;
             for (int i = 0; i < h.darks; i++) {
                 doff.push_back((int64_t)(fb * (size_t)i));
-                st = h2d_staged(p->d_dark_raw + doff.back(), b + off[(size_t)i], fb, p->stream);
+                st = h2d_staged(p, p->d_dark_raw + doff.back(), b + off[(size_t)i], fb);
                 if (st) return st;
             }
         }
@@ -767,7 +770,7 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
     const size_t pad = 256;
     st = reserve(&p->d_imm_owned, &p->imm_cap, len + pad);
     if (st) return st;
-    st = h2d_staged(p->d_imm_owned, b + lo, len, p->stream);
+    st = h2d_staged(p, p->d_imm_owned, b + lo, len);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
     std::vector<int64_t> so(sel.size());
@@ -840,7 +843,7 @@ extern "C" xpcs_status xpcs_mt_ingest_events(xpcs_mt_plan* p, const int32_t* pix
     const size_t pad = 256;
     st = reserve(&p->d_imm_owned, &p->imm_cap, bytes + pad);
     if (st) return st;
-    st = h2d_staged(p->d_imm_owned, buf.data(), bytes, p->stream);
+    st = h2d_staged(p, p->d_imm_owned, buf.data(), bytes);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
     st = finish_selection(p, so, sd, ofr);
@@ -942,7 +945,7 @@ extern "C" xpcs_status xpcs_mt_ingest_packed(xpcs_mt_plan* p, const void* words,
     const size_t len = (size_t)(hi - lo) * (size_t)wb;
     st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
     if (st) return st;
-    st = h2d_staged(p->d_imm_owned, static_cast<const uint8_t*>(words) + (size_t)lo * (size_t)wb, len, p->stream);
+    st = h2d_staged(p, p->d_imm_owned, static_cast<const uint8_t*>(words) + (size_t)lo * (size_t)wb, len);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
     std::vector<int64_t> so(rec.size());
@@ -992,7 +995,7 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
     st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
     if (st) return st;
     if (bytes_per_value == 2) {
-        st = h2d_staged(p->d_imm_owned, static_cast<const uint8_t*>(frames) + (size_t)f_lo * npd * 2, len, p->stream);
+        st = h2d_staged(p, p->d_imm_owned, static_cast<const uint8_t*>(frames) + (size_t)f_lo * npd * 2, len);
     } else {
         // 32-bit values narrowed on the host (the kernels read 16-bit values)
         const uint32_t* src = static_cast<const uint32_t*>(frames) + (size_t)f_lo * npd;
@@ -1003,7 +1006,7 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
                             (long long)(f_lo + (int64_t)(i / (size_t)npd)));
             nar[i] = (uint16_t)src[i];
         }
-        st = h2d_staged(p->d_imm_owned, reinterpret_cast<const uint8_t*>(nar.data()), len, p->stream);
+        st = h2d_staged(p, p->d_imm_owned, reinterpret_cast<const uint8_t*>(nar.data()), len);
     }
     if (st) return st;
     p->d_imm = p->d_imm_owned;
@@ -1254,7 +1257,7 @@ static xpcs_status read_ipif(xpcs_mt_plan* p, const int64_t* d, int64_t* out)
 {
     const size_t n = (size_t)p->h.P * p->h.T;
     if (!p->ipif32) {
-        return d2h_staged(out, d, n * sizeof(int64_t), p->stream);
+        return d2h_staged(p, out, d, n * sizeof(int64_t));
     }
     std::vector<uint32_t> w(2 * n);
     std::vector<uint64_t> tot((size_t)p->h.P);
@@ -1304,7 +1307,7 @@ extern "C" xpcs_status xpcs_mt_read_sums_i64(xpcs_mt_plan* p, int64_t* G2, int64
     if (st) return st;
     const size_t n = (size_t)p->h.P * p->h.T * sizeof(int64_t);
     if (G2) {
-        st = d2h_staged(G2, p->d_G2, n, p->stream);
+        st = d2h_staged(p, G2, p->d_G2, n);
         if (st) return st;
     }
     if (IP && (st = read_ipif(p, p->d_IP, IP))) return st;

@@ -367,7 +367,7 @@ int tt_diag_segments(int32_t F);
 void launch_tt_diag(xpcs_mt_plan* p, double* C, int32_t F, int32_t wsize, int32_t total, double rescale,
                     double* partial, double* g2full, double* g2part, hipStream_t s);
 void twotime_release(xpcs_mt_plan* p);
-xpcs_status d2h_staged(void* dst, const void* src, size_t len, hipStream_t s);
+xpcs_status d2h_staged(xpcs_mt_plan* p, void* dst, const void* src, size_t len);
 
 // online multi-tau (k_stream.hip)
 constexpr int kStreamChunk = 64;   // frames per update launch

@@ -363,7 +363,7 @@ extern "C" xpcs_status xpcs_mt_read_twotime(xpcs_mt_plan* p, int32_t i, double* 
     if (!p || !c2t) return fail(XPCS_ERR_INVALID_ARG, "read_twotime: NULL argument");
     if (i < 0 || i >= (int32_t)p->tt_c2t.size()) return fail(XPCS_ERR_RANGE, "read_twotime: no q-bin %d", i);
     const size_t F = (size_t)p->h.F;
-    return d2h_staged(c2t, p->tt_c2t[(size_t)i], sizeof(double) * F * F, p->stream);
+    return d2h_staged(p, c2t, p->tt_c2t[(size_t)i], sizeof(double) * F * F);
 }
 
 extern "C" xpcs_status xpcs_mt_read_twotime_1d(xpcs_mt_plan* p, double* g2full, double* g2partials, double* sg)
