@@ -1,5 +1,7 @@
-"""Large results read by several threads, and with another device current."""
+"""Large results read while other threads use the library, and with another
+device current."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -23,6 +25,39 @@ def executed(xmt, W, F, seed):
 
 def read_into(xmt, plan, out):
     xmt.check(xmt.lib().xpcs_mt_read_sums_i64(plan._h, xmt._p(out), None, None))
+
+
+def test_reads_during_an_ingest(xmt):
+    """A read of megabytes does not wait for another thread's upload."""
+    reader, G2 = executed(xmt, 256, 200, 1)
+    assert G2.nbytes > 8 << 20
+    W, F = 512, 6000          # 3 GB of frames, more than 50 ms of upload
+    ones = np.ones((W, W), np.int32)
+    big = xmt.Plan(W, W, F, 4, ones, ones)
+    frames = np.zeros((F, W * W), np.uint16)
+    out = np.empty_like(G2)
+    read_into(xmt, reader, out)                # buffers made, pages touched
+    span = []
+
+    def ingest():
+        t = time.perf_counter()
+        big.ingest_frames(frames)
+        span.extend([t, time.perf_counter()])
+    th = threading.Thread(target=ingest)
+    reads = []
+    th.start()
+    while th.is_alive():
+        out[:] = -1
+        t = time.perf_counter()
+        read_into(xmt, reader, out)
+        reads.append((t, time.perf_counter()))
+        assert np.array_equal(out, G2)
+    th.join()
+    inside = [r for r in reads if r[0] > span[0] and r[1] < span[1]]
+    print(f"upload {1e3 * (span[1] - span[0]):.0f} ms, {len(inside)} reads within", flush=True)
+    big.close()
+    reader.close()
+    assert len(inside) >= 3
 
 
 def test_reads_of_several_threads(xmt):

@@ -533,9 +533,9 @@ xpcs_status finish_selection(xpcs_mt_plan* p, const std::vector<int64_t>& sel_of
     return XPCS_OK;
 }
 
-// Two pinned buffers and the events of the last copy through each.  A device
-// has one pool, made on first use, which lives until the process ends and is
-// shared by the device's plans (one staged copy at a time).
+// Two pinned buffers and the events of the last copy through each.  Uploads and
+// reads have a pool each per device, made on first use, which lives until the
+// process ends and is shared by the device's plans.
 struct StagePool {
     std::mutex mu;
     uint8_t* buf[2] = {nullptr, nullptr};
@@ -546,10 +546,10 @@ constexpr size_t kStageUpload = size_t(32) << 20;
 constexpr size_t kStageRead = size_t(8) << 20;
 
 // The pool of the plan's device, whichever device is current.
-StagePool& stage_pool(const xpcs_mt_plan* p)
+StagePool& stage_pool(const xpcs_mt_plan* p, bool read)
 {
-    static StagePool pools[64];   // eight GPUs of eight partitions
-    return pools[p->device & 63];
+    static StagePool pools[2][64];   // eight GPUs of eight partitions
+    return pools[read][p->device & 63];
 }
 
 // The pool's buffers of `bytes` and its events, made on first use (sp.mu held).
@@ -600,7 +600,7 @@ void parallel_copy(uint8_t* dst, const uint8_t* src, size_t n)
 xpcs_status h2d_staged(xpcs_mt_plan* p, uint8_t* dst, const uint8_t* src, size_t len)
 {
     if (len == 0) return XPCS_OK;
-    StagePool& sp = stage_pool(p);
+    StagePool& sp = stage_pool(p, false);
     std::lock_guard<std::mutex> lk(sp.mu);
     xpcs_status st = stage_ready(sp, p->device, kStageUpload);
     if (st) return st;
@@ -668,20 +668,21 @@ namespace xpcs {
 // stream.  Large ones come through the pinned buffers a piece at a time, one
 // piece on the link while threads copy the other out (a plain copy ran at 13
 // GB/s, most of it first-touch page faults of the caller's array on one
-// thread).
+// thread).  A plain copy where the buffers cannot be had, or another thread's
+// read has them.
 xpcs_status d2h_staged(xpcs_mt_plan* p, void* dst, const void* src, size_t len)
 {
     if (len == 0) return XPCS_OK;
     hipStream_t s = p->stream;
-    if (len < (size_t(2) << 20)) {
+    StagePool& sp = stage_pool(p, true);
+    std::unique_lock<std::mutex> lk(sp.mu, std::defer_lock);
+    if (len < (size_t(2) << 20) || !lk.try_lock() || stage_ready(sp, p->device, kStageRead) != XPCS_OK) {
+        (void)hipGetLastError();   // of a failed pinned allocation
         HIP_TRY(hipMemcpyAsync(dst, src, len, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         return XPCS_OK;
     }
-    StagePool& sp = stage_pool(p);
-    std::lock_guard<std::mutex> lk(sp.mu);
-    xpcs_status st = stage_ready(sp, p->device, kStageUpload);
-    if (st) return st;
+    xpcs_status st = XPCS_OK;
     uint8_t* d = static_cast<uint8_t*>(dst);
     const uint8_t* q = static_cast<const uint8_t*>(src);
     const size_t pieces = (len + kStageRead - 1) / kStageRead;
