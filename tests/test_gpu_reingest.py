@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import cases
+import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -40,4 +41,60 @@ def test_rows_then_fewer_imm_events(xmt, orc, first):
         plan.ingest_imm(c["imm"])
         plan.execute()
         check(plan, orc.run_exact(c["imm"], c["dq"], c["sq"], c["F"], c["dpl"]))
+    plan.close()
+
+
+def busy_stream():
+    """A torch stream with a tenth of a second of work queued."""
+    import torch
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(200_000_000)
+    return s
+
+
+INGESTS = {
+    "imm": lambda xmt, plan, c, W, H: plan.ingest_imm(synth.imm_bytes_sparse(c, W, H)),
+    "dense": lambda xmt, plan, c, W, H: plan.ingest_imm(synth.imm_bytes_dense(c, W, H)),
+    "frames": lambda xmt, plan, c, W, H: plan.ingest_frames(c),
+    "rows": lambda xmt, plan, c, W, H: plan.ingest_rows(*rows_of(c)),
+    "ufxc": lambda xmt, plan, c, W, H: plan.ingest_packed(synth.ufxc_words(c, W, H), xmt.FMT_UFXC),
+    "events": lambda xmt, plan, c, W, H: plan.ingest_events(
+        np.nonzero(c)[1].astype(np.int32), c[np.nonzero(c)].astype(np.uint16),
+        np.concatenate([[0], np.cumsum((c > 0).sum(1))]).astype(np.int64)),
+}
+
+
+@pytest.mark.parametrize("batch", [False, True])
+@pytest.mark.parametrize("kind", sorted(INGESTS))
+def test_ingest_waits_for_a_callers_stream(xmt, orc, kind, batch):
+    """The plan's previous data is still to be read by work on another stream
+    when the next data is handed in: the ingest waits for it, and the sums are
+    the new data's."""
+    import torch
+    W, H, F = 32, 24, 150
+    dq, sq = synth.annular_qmaps(W, H, 6, 3)
+    data = [np.minimum(synth.ou_counts(W, H, F, 0.2, 8.0, seed=k), 3).astype(np.uint16) for k in (1, 2, 3)]
+    plan = xmt.Plan(W, H, F, 4, dq, sq)
+    ingest = INGESTS[kind]
+    ingest(xmt, plan, data[0], W, H)
+    plan.execute()
+    plan.sums()
+    jobs = xmt.Batch()
+    if batch:
+        jobs.add(plan)
+        jobs.execute()
+        jobs.synchronize()
+    for c in data[1:]:
+        print("ingest after work on another stream:", kind, batch, flush=True)
+        s = busy_stream()
+        (jobs if batch else plan).execute(stream=s.cuda_stream)
+        done = s.record_event()
+        assert not done.query()
+        ingest(xmt, plan, c, W, H)
+        assert done.query()
+        plan.execute()
+        check(plan, orc.run_exact(synth.imm_bytes_sparse(c, W, H), dq, sq, F, 4))
+    torch.cuda.synchronize()
+    jobs.close()
     plan.close()
