@@ -58,7 +58,7 @@ def sparse_kernel_bytes(T, E_raw, nsel, nrows, n_mapped, tuning, px, ev, tdeep=N
     the deep taus of those rows."""
     P = int(px.sum())
     E0 = int(ev.sum())
-    bshift = int(tuning["tr_bucket_shift"])
+    bshift = int(tuning["tr_bucket_shift"]) or 7   # 0: the automatic choice of 2^7
     nb = (nrows + (1 << bshift) - 1) >> bshift
     cf = int(tuning["tr_chunk_frames"])
     nh = nb * max(1, (nsel + cf - 1) // cf)
