@@ -352,8 +352,10 @@ xpcs_status xpcs_mt_set_timing_filter(xpcs_mt_plan* plan, const char* name);
  *   tr_bucket_shift  pixels per transpose bucket = 2^shift (8..12; 0 from
  *                    get_tuning: the automatic choice is 2^7)
  *   tr_chunk_frames  raw frames per transpose workgroup (>= 1)
- *   reg_blocks       workgroups of the register-resident row kernel (1..65535)
- *   lds_blocks       workgroups of the LDS row kernel (1..65535)
+ *   reg_blocks       workgroups of the kernel of rows of at most 64 events
+ *                    (1..65535; 0 from get_tuning: as many as the rows need)
+ *   lds_blocks       workgroups of the kernels of longer rows (1..65535; 0 from
+ *                    get_tuning: each kernel's own number)
  *   dense_levels     levels per pass of the dense streaming kernel, i.e. the
  *                    depth of its register-resident lag window
  *                    (dpl 4: 3, 4, 5; dpl 8: 2, 3)
@@ -480,8 +482,10 @@ xpcs_status xpcs_mt_stream_open(const xpcs_mt_desc* desc, int32_t max_frames, xp
 /* Whole compressed IMM frames in host memory (free again on return). */
 xpcs_status xpcs_mt_stream_push_imm(xpcs_mt_stream* stream, const void* imm, size_t nbytes);
 /* Frames already in device memory: payload offsets / event counts per frame
- * (host arrays); the device bytes must stay valid until the next snapshot
- * has finished. */
+ * (host arrays).  The frames are read on the stream's own HIP stream, which
+ * waits for no other: what writes them must have completed before the call
+ * (xpcs_mt_ingest_imm_device, once per job, waits for the device itself), and
+ * the device bytes must stay valid until the next snapshot has finished. */
 xpcs_status xpcs_mt_stream_push_imm_device(xpcs_mt_stream* stream, const void* dev_imm, size_t nbytes,
                                            const int64_t* payload_off, const uint32_t* dlen, int32_t nframes);
 /* Frames pushed so far and the taus of their schedule. */

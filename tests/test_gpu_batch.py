@@ -133,6 +133,20 @@ def test_sparse_shapes_keep_results(xmt, shapes):
     assert_same(results(p), want)
 
 
+@pytest.mark.parametrize("dpl,rows", [(8, True), (5, False)])
+def test_tuning_as_reported(xmt, dpl, rows):
+    """Automatic shapes of the row kernels are reported as automatic, those of
+    the other kernels as launched; set again as reported, they are the same."""
+    c = cases.sparse_case(W=40, H=40, F=1300, dpl=dpl, mu=0.3, tau_c=20.0, seed=81, S=8, Q=4)
+    p = make_plan(xmt, c)
+    t = p.get_tuning()
+    assert (t["reg_blocks"], t["lds_blocks"]) == ((0, 0) if rows else ((p.P + 7) // 8, 2048))
+    p.set_tuning(**t)
+    assert p.get_tuning() == t
+    p.set_tuning(reg_blocks=3, lds_blocks=5)
+    assert (p.get_tuning()["reg_blocks"], p.get_tuning()["lds_blocks"]) == (3, 5)
+
+
 @pytest.mark.parametrize("dpl,levels", [(4, 3), (4, 5), (8, 2)])
 def test_dense_levels_keep_results(xmt, orc, dpl, levels):
     c = dense_case(16, 12, 1500, dpl, 2.0, 15.0, seed=83 + levels)

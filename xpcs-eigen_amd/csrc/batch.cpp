@@ -92,10 +92,13 @@ extern "C" xpcs_status xpcs_mt_get_tuning(xpcs_mt_plan* p, xpcs_mt_tuning* t)
                                               p->raw_events, p->tune.tr_bucket_shift, p->tune.tr_chunk_frames);
     t->tr_bucket_shift = sh.bshift >= 8 ? sh.bshift : 0;   // 2^7 is the automatic choice's alone
     t->tr_chunk_frames = (int32_t)sh.cf;
-    t->reg_blocks = reg_blocks(p);
-    t->lds_blocks = lds_blocks(p);
+    // the row kernels' automatic grids differ by length class (as many
+    // workgroups as the rows need, 4096 for the lists) and may pass 65535: 0
+    const bool rows = p->mode != 2 && rows_supported(p);
+    t->reg_blocks = rows ? p->tune.reg_blocks : reg_blocks(p);
+    t->lds_blocks = rows ? p->tune.lds_blocks : lds_blocks(p);
     t->dense_levels = (p->h.dpl == 4 || p->h.dpl == 8) ? dense_levels(p) : 0;
-    t->deep_frames = p->tune.deep_frames < 0 ? -1 : (p->tune.deep_frames > 0 ? p->tune.deep_frames : rows_supported(p) ? 0 : 96);
+    t->deep_frames = p->tune.deep_frames < 0 ? -1 : (p->tune.deep_frames > 0 ? p->tune.deep_frames : rows ? 0 : 96);
     t->sums64 = p->tune.sums64;
     return XPCS_OK;
 }
@@ -147,8 +150,9 @@ extern "C" xpcs_status xpcs_mt_autotune(xpcs_mt_plan* p, xpcs_mt_tuning* best_ou
         }
         axes.push_back({&xpcs_mt_tuning::reg_blocks, {1024, 4096}});
         axes.push_back({&xpcs_mt_tuning::lds_blocks, {256, 2048, 4096, 8192}});
-        // deep-level hand-over: none, or from the first level with <= 48 frames
-        // (the default is <= 96)
+        // dense series: none, or from the first level with <= 48 frames (the
+        // default: three frames per event of the row kernels' length class, 96
+        // in the other kernels)
         int dstride = 0;
         if (deep_level(p, &dstride) < (int)p->h.levels.size())
             axes.push_back({&xpcs_mt_tuning::deep_frames, {-1, 48}});

@@ -548,6 +548,8 @@ class Stream:
         check(lib().xpcs_mt_stream_push_imm(self._h, _p(b), b.size))
 
     def push_imm_device(self, ptr, nbytes, payload_off, dlen):
+        """Frames in device memory, completely written before the call (it
+        waits for no other stream) and kept until the next snapshot is done."""
         off = np.ascontiguousarray(payload_off, np.int64)
         dl = np.ascontiguousarray(dlen, np.uint32)
         check(lib().xpcs_mt_stream_push_imm_device(self._h, C.c_void_p(ptr), nbytes, _p(off), _p(dl), off.size))
