@@ -40,3 +40,37 @@ def test_dense_dot_sums(xmt, orc, W, H, dpl, F, darks, scale):
     r = orc.run_exact(imm, dq, sq, F, dpl, **kw)
     assert np.array_equal(a, r["IP"]) and np.array_equal(b, r["IF"])
     assert np.array_equal(g, r["G2"])
+
+
+def test_buffers_of_a_short_run(xmt):
+    """A short run on a large detector holds its boundary sums once, beside the
+    first series."""
+    torch = pytest.importorskip("torch")
+    W, F, dpl = 1024, 64, 4
+    ones = np.ones((W, W), np.int32)
+    frames = np.ones((F, W * W), np.uint16)
+    small = xmt.Plan(64, 64, F, dpl, ones[:64, :64], ones[:64, :64])   # the kernels' own memory first
+    small.ingest_frames(frames[:, :64 * 64])
+    small.execute()
+    small.sums()
+    plan = xmt.Plan(W, W, F, dpl, ones, ones)
+    plan.ingest_frames(frames)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan.execute()
+    plan.synchronize()
+    used = free - torch.cuda.mem_get_info()[0]
+    levels, taus = xmt.delays_per_level(F, dpl)
+    bounds = set()
+    for L, tau in zip(levels, taus):
+        lf, t = F >> L, int(tau) >> L
+        bounds |= {(lf - t) << L, t << L, lf << L}
+    need = 4 * W * W * (len(bounds) + (F >> 4))
+    print(f"buffers {used >> 20} MiB for {need >> 20}", flush=True)
+    g, a, b = plan.sums()
+    plan.close()
+    small.close()
+    assert used < 1.25 * need
+    n = np.array([(F >> L) - (int(t) >> L) for L, t in zip(levels, taus)])
+    assert (a[0] == n << levels).all() and (a == a[0]).all() and (b == a[0]).all()
+    assert (g == (n << levels) << levels).all()

@@ -1153,9 +1153,8 @@ xpcs_status prepare_execute(xpcs_mt_plan* p)
             xpcs_status st = dalloc(&p->d_wave_flags, ((size_t)h.W * h.H + 255) / 256 * 4);
             if (st) return st;
         }
-        const size_t need = dense_series_elems(p);
-        xpcs_status st = reserve(&p->d_series_a, &p->series_a_cap, need);
-        if (!st) st = reserve(&p->d_series_b, &p->series_b_cap, need);
+        xpcs_status st = reserve(&p->d_series_a, &p->series_a_cap, dense_series_elems(p, 0));
+        if (!st) st = reserve(&p->d_series_b, &p->series_b_cap, dense_series_elems(p, 1));
         if (st) return st;
     } else if (p->mode == 2) {
         const xpcs_status st = reserve(&p->d_rows, &p->rows_cap, (size_t)h.P * (size_t)h.F);

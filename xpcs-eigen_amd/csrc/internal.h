@@ -315,7 +315,7 @@ void launch_mt_long(xpcs_mt_plan* p, hipStream_t s, bool dense_rows);
 void launch_dense_transpose(xpcs_mt_plan* p, hipStream_t s);
 void launch_side(xpcs_mt_plan* p, hipStream_t s);
 bool dense_stream_supported(const HostTables& h);
-size_t dense_series_elems(const xpcs_mt_plan* p);
+size_t dense_series_elems(const xpcs_mt_plan* p, int which);
 int dense_levels(const xpcs_mt_plan* p);
 bool dense_levels_allowed(int dpl, int k);
 int reg_blocks(const xpcs_mt_plan* p);

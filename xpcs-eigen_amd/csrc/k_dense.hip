@@ -1177,15 +1177,17 @@ static bool dense_dot_ok(const xpcs_mt_plan* p)
     return !p->fsnorm && p->even_off0 >= 0 && p->h.avg == 1 && (int64_t)p->h.W * p->h.H >= 8 && p->nscale <= 1024 && p->d_wave_flags;
 }
 
-size_t dense_series_elems(const xpcs_mt_plan* p)
+// 32-bit words of the two series buffers: the first pass writes the first one,
+// the next the second, and so on; level values as u32, or frame-weighted as
+// FP64 (2 words).  The first pass also keeps its boundary sums in the second.
+size_t dense_series_elems(const xpcs_mt_plan* p, int which)
 {
     const HostTables& h = p->h;
-    const size_t K = (size_t)dense_levels(p);
-    // 32-bit words: u32 level values, or FP64 frame-weighted values (2 words)
+    const size_t npd = (size_t)h.W * (size_t)h.H;
+    const size_t L = (size_t)dense_levels(p) * (size_t)(which + 1);   // first level that the buffer holds
     const size_t words = p->fsnorm ? 2 : 1;
-    const size_t series = h.levels.size() > K ? words * (size_t)h.levels[K].lf * (size_t)h.W * (size_t)h.H : 1;
-    // the first pass keeps its boundary sums in the second buffer
-    return std::max(series, dense_dot_ok(p) ? (size_t)p->nrank * (size_t)h.W * (size_t)h.H : (size_t)1);
+    const size_t series = h.levels.size() > L ? words * (size_t)h.levels[L].lf * npd : 1;
+    return std::max(series, which == 1 && dense_dot_ok(p) ? (size_t)p->nrank * npd : (size_t)1);
 }
 
 template <int DPL, int K>
