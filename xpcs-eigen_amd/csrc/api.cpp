@@ -55,18 +55,6 @@ static xpcs_status reserve(T** p, size_t* cap, size_t n)
     return st;
 }
 
-template <typename T>
-static xpcs_status upload(T** p, const std::vector<T>& v, hipStream_t s)
-{
-    xpcs_status st = dalloc(p, v.size());
-    if (st) return st;
-    if (!v.empty()) {
-        hipError_t e = hipMemcpyAsync(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) return fail(XPCS_ERR_HIP, "upload: %s", hipGetErrorString(e));
-    }
-    return XPCS_OK;
-}
-
 // One device allocation for everything a plan holds from its creation: the
 // tables first (one host image, one copy), then the buffers.  Thirty separate
 // allocations and copies took 2 ms of opening a 256 x 256 stream.
