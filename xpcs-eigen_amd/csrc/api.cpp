@@ -475,10 +475,12 @@ xpcs_status dense_prepare(xpcs_mt_plan* p, const uint8_t* base, const std::vecto
     HostTables& h = p->h;
     p->nscale = h.darks > 0 ? h.darks : 1;
     xpcs_status st = XPCS_OK;
+    const bool made = !p->d_dark_sum || !p->d_thr;
     if (!p->d_dark_sum) st = dalloc(&p->d_dark_sum, (size_t)h.P);
     if (!st && !p->d_thr) st = dalloc(&p->d_thr, (size_t)h.P);
     if (st) return st;
     if (h.darks == 0) {
+        if (!made) return XPCS_OK;   // zeros for the plan's lifetime
         launch_fill_u64(reinterpret_cast<uint64_t*>(p->d_dark_sum), (size_t)h.P, p->stream);
         launch_fill_u64(reinterpret_cast<uint64_t*>(p->d_thr), (size_t)h.P, p->stream);
     } else {

@@ -237,7 +237,7 @@ struct xpcs_mt_plan {
     size_t wide_flags_cap = 0;
     uint32_t* d_counters = nullptr;      // in d_stat: [0] rows over 1024 events, [1] error flags, [2] rows of 65..128,
                                          // [3] dense exact-redo pixels, [4] rows of 129..512, [5] 513..1024,
-                                         // [6] rows in d_wide_list, [7] some row is flagged in d_wide_flags
+                                         // [6] rows in d_wide_list, [7] some row is flagged in d_wide_flags, or dense waves flagged by k_dense_look
     uint32_t* d_deep = nullptr;          // [P][deep stride] level series handed to the one-lane-per-pixel kernel
     size_t deep_cap = 0;
     uint64_t* d_scratch = nullptr;

@@ -433,21 +433,21 @@ k_mt_dense_f64(const uint8_t* __restrict__ imm, const int64_t* __restrict__ sel_
 // multiply-adds, the pair sums and the running total are dot products with
 // (1, 1), and dark subtraction and threshold work on both halves at once.
 //
-// Lag sums run in 32 bits and are added to the FP64 totals (flush) before they
-// could overflow: a chunk between flushes holds at most kDotChunk counts per
-// pixel, the 68 frames before it (five groups, the deepest lag) at most five
-// times that, and kDotChunk (kDotChunk + 5 kDotChunk) < 2^32; kDotChunk also
-// keeps every value of a group's levels in 16 bits.  A wave that meets a
-// 16-frame group beyond kDotChunk in any pixel flags its 64 pixels and stops;
-// the FP64 kernel then takes exactly those.
+// Lag sums run in 32 bits and are added to 64-bit totals (flush) before they
+// could overflow: between flushes a pixel counts at most `chunk` (kDotChunk, or
+// half of it), each of those counts meets one value per lag, and values have 16
+// bits, so a lag sum is at most kDotChunk 65535 < 2^32.  That also keeps every
+// value of a group's levels in 16 bits.  A wave that meets a 16-frame group
+// beyond `chunk` in any pixel flags its 64 pixels and stops; the FP64 kernel
+// then takes exactly those.
 //
 // The FP64 form was bound by vector issue (20 instructions per frame and
 // wave, two waves per SIMD); measured on the 512 x 512 x 20,000-frame job
 // (dpl 4, two darks): 3.45 -> 2.58 ms (11 GB of HBM traffic, 4.3 TB/s: memory
 // now bounds it), on 333 x 251 x 3001 frames (dpl 8) 1.04 -> 0.36 ms.
-constexpr uint32_t kDotChunk = 26000u;
-using u16x2 = __attribute__((ext_vector_type(2))) unsigned short;
+constexpr uint32_t kDotChunk = 64500u;
 using i16x2 = __attribute__((ext_vector_type(2))) short;
+using u16x2 = __attribute__((ext_vector_type(2))) unsigned short;
 
 __device__ __forceinline__ uint32_t dot2_u16(uint32_t a, uint32_t b, uint32_t c)
 {
@@ -528,7 +528,7 @@ struct DotArgs {
     const uint8_t* src;           // payload of frame t at src + t * step
     int64_t step;
     const int32_t* pix2c;
-    uint32_t npix, n_in;
+    uint32_t npix, n_in, chunk;
     const int64_t* dark_sum;
     const int64_t* thr;
     int32_t nscale;
@@ -547,8 +547,52 @@ struct DotArgs {
     uint32_t* redo_count;
     int32_t* redo_list;
     uint32_t* wave_flags;         // per 64 pixels: left to the FP64 kernel
+    const uint32_t* bright;       // waves that k_dense_look flagged; NULL: it has not run
+    uint32_t most;                // beyond so many of them all are left to the FP64 kernel
     bool w32;
 };
+
+// A look at groups across the run before the dot kernel: a wave with one above
+// two thirds of the chunk is likely to pass it somewhere, and would then have
+// walked its frames for nothing.  Flags such waves and counts them.  Speckle
+// frames of a mean of 300 (900) counts, 333 x 251 x 3001, dpl 8: 1.54 (1.34) ->
+// 1.24 (1.25) ms, the FP64 kernel's own time, where the dot kernel alone had
+// taken waves to their first group beyond 26000; of 300 scaled counts, 512 x
+// 512 x 6000 with two darks, dpl 4: 2.0 -> 1.65 ms; of 600: 1.74 -> 1.42 ms.  The
+// look takes 7 to 10 us.
+constexpr uint32_t kDotLookFrames = 1024u;   // shorter runs: not worth a launch
+constexpr int kLookGroups = 4;
+
+__global__ void __launch_bounds__(256)
+k_dense_look(const uint8_t* __restrict__ src, int64_t step, const int32_t* __restrict__ pix2c, uint32_t npix,
+             uint32_t n_in, const int64_t* __restrict__ dark_sum, const int64_t* __restrict__ thr, int32_t nscale,
+             uint32_t limit, uint32_t* __restrict__ wave_flags, uint32_t* __restrict__ bright)
+{
+    const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
+    const int32_t c = gid < npix ? pix2c[gid] : -1;
+    bool hit = false;
+    if (c >= 0) {
+        const int32_t nds = -(int32_t)dark_sum[c];
+        const int64_t t = thr[c];
+        const int32_t th = t < 0 ? 0 : (t > INT32_MAX ? INT32_MAX : (int32_t)t);
+        const uint8_t* col = src + 2 * (int64_t)gid;
+#pragma unroll
+        for (int g = 0; g < kLookGroups; g++) {
+            const uint32_t t0 = n_in / kGroup * (2u * (uint32_t)g + 1u) / (2u * kLookGroups) * kGroup;
+            uint32_t sum = 0u;
+#pragma unroll
+            for (int u = 0; u < kGroup; u++)
+                sum += dense_value(*reinterpret_cast<const uint16_t*>(col + (int64_t)(t0 + (uint32_t)u) * step), nscale, nds, th);
+            hit |= sum > limit;
+        }
+    }
+    const uint64_t m = __ballot(hit);
+    if ((threadIdx.x & 63u) == 0u && gid < npix) {
+        wave_flags[gid >> 6] = m != 0ull;
+        if (m != 0ull) atomicAdd(bright, 1u);
+    }
+}
+
 
 struct __attribute__((packed, aligned(2))) Raw8 {
     uint32_t w[4];
@@ -557,7 +601,9 @@ struct __attribute__((packed, aligned(2))) Raw8 {
 // DARK: n-scaled values y = n raw - sum(dark), kept iff y > max(threshold, 0):
 // with m = floor((max(threshold, 0) + sum(dark)) / n) and t = max(raw - m, 0)
 // that is t > 0 and y = n t + (n m - sum(dark)).  t is limited so that y fits
-// 16 bits; a limited value alone passes kDotChunk.
+// 16 bits (a limited value is above 65535 - n, n at most 1024) and t 15: with
+// n >= 2 that limits no further, with n = 1 to 32767, and `chunk` is below that.
+// So a limited value alone passes `chunk`.
 //
 // W neighbouring waves to a workgroup and two waves per SIMD: more waves in
 // flight scatter the frame reads (512 x 512 x 20,000 frames, dpl 4: 2.58 ms
@@ -582,15 +628,17 @@ k_mt_dense_dot(const DotArgs a)
     const uint32_t n_in = a.n_in;
     const int32_t c = gid < a.npix ? a.pix2c[gid] : -1;
     const bool active = c >= 0;
-    if (lane == 0 && gid < a.npix) a.wave_flags[gid >> 6] = 0u;
     if (__ballot(active) == 0ull) return;
+    const bool left = a.bright && (*a.bright > a.most || a.wave_flags[gid >> 6] != 0u);
+    if (lane == 0) a.wave_flags[gid >> 6] = left;
+    if (left) return;
     uint32_t rm = 0u, c0 = 0u, tlim = 0u, nsc = 0u;   // in both halves
     if constexpr (DARK) {
         const int64_t n = a.nscale;
         const int64_t ds = active ? a.dark_sum[c] : 0;
         const int64_t th = active ? a.thr[c] : 0;
         const int64_t m = min(((th < 0 ? 0 : th) + ds) / n, (int64_t)65535);
-        int64_t k0 = n * m - ds, tl = min((int64_t)32767, (65535 - (k0 > 0 ? k0 : 0)) / n), sc = n;
+        int64_t k0 = n * m - ds, tl = min((int64_t)32767, (65535 - k0) / n), sc = n;
         if (tl < 1) {
             // the smallest kept value passes 16 bits: any kept value ends the wave
             k0 = 65535;
@@ -632,7 +680,7 @@ k_mt_dense_dot(const DotArgs a)
     };
     while (cur == 0) capture(0u);   // a boundary at frame 0 covers no frames
 
-    // one group; `over` once a pixel of the wave has passed kDotChunk (what the
+    // one group; `over` once a pixel of the wave has passed the chunk (what the
     // group then adds is not used)
     bool over = false;
     auto group = [&](const uint32_t (&raw)[8], uint32_t t0, auto tail) {
@@ -660,7 +708,7 @@ k_mt_dense_dot(const DotArgs a)
 #pragma unroll
         for (int i = 0; i < 2; i++) x2[i] = pair_up(x1[2 * i], x1[2 * i + 1]);
         x3[0] = pair_up(x2[0], x2[1]);
-        // the group's sum (saturated halves pass kDotChunk)
+        // the group's sum (saturated halves pass the chunk)
         const uint32_t gs = (x3[0] & 0xFFFFu) + (x3[0] >> 16);
         if constexpr (TAIL) {
             // values past the end of their level do not exist in its series
@@ -677,8 +725,8 @@ k_mt_dense_dot(const DotArgs a)
             x3[0] = pair_up(x2[0], x2[1]);
             cut(x3, 1, 3);
         }
-        if (__ballot(active && S + gs - S0 > kDotChunk) != 0ull) {
-            over = over || __ballot(active && gs > kDotChunk) != 0ull;
+        if (__ballot(active && S + gs - S0 > a.chunk) != 0ull) {
+            over = over || __ballot(active && gs > a.chunk) != 0ull;
             dot_flush<DPL, K>(s, tot);
             S0 = S;
         }
@@ -1201,6 +1249,7 @@ static void launch_dense_dot(xpcs_mt_plan* p, hipStream_t s, int nlev_pass, uint
     a.pix2c = p->d_pix2c;
     a.npix = (uint32_t)(h.W * h.H);
     a.n_in = (uint32_t)h.F;
+    a.chunk = h.darks == 1 ? kDotChunk / 2 : kDotChunk;
     a.dark_sum = p->d_dark_sum;
     a.thr = p->d_thr;
     a.nscale = (int32_t)p->nscale;
@@ -1220,6 +1269,18 @@ static void launch_dense_dot(xpcs_mt_plan* p, hipStream_t s, int nlev_pass, uint
     a.redo_count = redo_count;
     a.redo_list = p->d_long_list;
     a.wave_flags = p->d_wave_flags;
+    if (a.n_in >= kDotLookFrames) {
+        uint32_t* const bright = p->d_counters + 7;
+        k_dense_look<<<(a.npix + 255) / 256, 256, 0, s>>>(a.src, a.step, a.pix2c, a.npix, a.n_in, a.dark_sum, a.thr,
+                                                          a.nscale, a.chunk / 3 * 2, a.wave_flags, bright);
+        a.bright = bright;
+        // this kernel takes 0.7 (dpl 4) or 0.36 (dpl 8) of the FP64 kernel's
+        // time, so with that share of the waves left to it one pass of both is
+        // slower; a detector of at most two waves per SIMD takes either
+        // kernel's time as soon as one wave runs it
+        const uint32_t waves = (a.npix + 63) / 64;
+        a.most = waves <= 2048 ? 0 : DPL == 4 ? waves / 4 : waves / 8 * 5;
+    }
     a.w32 = p->ipif32;
     auto go = [&](auto waves) {
         constexpr int W = decltype(waves)::value;
