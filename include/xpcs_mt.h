@@ -363,9 +363,9 @@ xpcs_status xpcs_mt_set_timing_filter(xpcs_mt_plan* plan, const char* name);
  *                    level with at most deep_frames binned frames (16..96;
  *                    negative: never; 0: three frames per event of the row's
  *                    length class).  Only for dpl 4 or 8, and for frames F with
- *                    F + (2 dpl + 1) 2^(L-1) <= 65535, L that first level (0:
- *                    the one of rows of 64 events, which allows 63,231 frames at
- *                    dpl 4 and 61,183 at dpl 8; fewer for small deep_frames).
+ *                    F + (2 dpl + 1) 2^(L-1) <= 65535, L that first level
+ *                    (automatic: rows of 64 events, which allows 63,231 frames
+ *                    at dpl 4 and 61,183 at dpl 8; fewer with small deep_frames).
  *                    Longer plans hand rows of at most 128 events over to a
  *                    kernel of their own there (0: 96; T <= 128 and at most 48
  *                    taus from that level on, otherwise no hand-over).

@@ -75,6 +75,16 @@ def test_wide_rows(xmt, orc, dpl, F, wide):
     check_rows(xmt, orc, 20, 17, F, dpl, *draw_rows(rng, 340, F, wide), True)
 
 
+@pytest.mark.parametrize("dpl", [4, 8])
+@pytest.mark.parametrize("F", [17, 32, 33, 96, 97, 192, 193, 768, 769, 1536, 1537, 3072, 3073])
+def test_series_from_level_0(xmt, orc, dpl, F):
+    """Frame counts around the limits below which a length class sums level 0
+    from its series too, rows with many events a frame among them."""
+    rng = np.random.default_rng([dpl, F])
+    print(f"level 0 series dpl={dpl} F={F}", flush=True)
+    check_rows(xmt, orc, 20, 17, F, dpl, *draw_rows(rng, 340, F, 0.3), True)
+
+
 @pytest.mark.parametrize("dpl,F,deep,row_kernels", [
     (4, 63231, 0, True), (4, 63232, 0, False), (8, 61183, 0, True), (8, 61184, 0, False),
     (8, 65535 - 17 * 512, 96, True), (8, 65536 - 17 * 512, 96, False),

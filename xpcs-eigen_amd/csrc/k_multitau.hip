@@ -801,8 +801,12 @@ constexpr int kClassifyPer = 8;      // pixels per thread of the classification 
 // order does not matter: every row writes only its own sums.
 __global__ void __launch_bounds__(256)
 k_mt_classify(const int64_t* __restrict__ off, const int32_t* __restrict__ rowmap, int32_t P, bool regs,
-              int32_t* __restrict__ mid_list, int32_t* __restrict__ long_list, uint32_t* __restrict__ counters)
+              int32_t* __restrict__ mid_list, int32_t* __restrict__ long_list, uint32_t* __restrict__ counters,
+              uint4* __restrict__ wide_flags, uint32_t nflags)
 {
+    // the row kernels' flags, 16 bytes a thread (two per row at most)
+    const uint32_t tid = blockIdx.x * 256u + threadIdx.x;
+    if (tid < nflags) wide_flags[tid] = make_uint4(0u, 0u, 0u, 0u);
     __shared__ uint32_t s_cnt[4];
     __shared__ uint32_t s_base[4];
     if (threadIdx.x < 4) s_cnt[threadIdx.x] = 0u;
@@ -1803,7 +1807,8 @@ static void launch_rows(xpcs_mt_plan* p, hipStream_t s, const char* t_reg, const
     timer_begin(p, s, "k_mt_classify");
     if (h.P > 0)
         k_mt_classify<<<(unsigned)((h.P + 256 * kClassifyPer - 1) / (256 * kClassifyPer)), 256, 0, s>>>(
-            p->d_off, p->d_rowmap, h.P, regs || rows, p->d_mid_list, p->d_long_list, p->d_counters);
+            p->d_off, p->d_rowmap, h.P, regs || rows, p->d_mid_list, p->d_long_list, p->d_counters,
+            reinterpret_cast<uint4*>(p->d_wide_flags), rows ? (uint32_t)(rows_wide_flags(p) / 16) : 0u);
     timer_end(p, s);
     if (rows) {
         launch_mt_rows(p, s);

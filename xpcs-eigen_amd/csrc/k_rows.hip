@@ -32,7 +32,12 @@
 //
 // Levels from ldeep on: the binned series as 16-bit pairs in LDS, the group's
 // lanes over time, lag sums by two-element dot products against a register
-// window, binning by adding a word's halves.
+// window, binning by adding a word's halves.  From level 0 on where the frames
+// are few for the row's events: with several events a frame, as averaging frames
+// leaves them, the pairs would be many times the series (256 x 256, dpl 8, whole
+// passes with the walk on level 0, with the series, and with a wave per row: 60
+// frames of 16 averaged, 480 events a row, 5.7, 0.69 and 1.29 ms; 200 of 4, 400
+// events, 1.98, 0.67 and 1.09 ms).
 #include <algorithm>
 #include <type_traits>
 
@@ -44,7 +49,7 @@ namespace xpcs {
 namespace {
 
 constexpr int kRowsWaves = 2;     // waves per workgroup
-constexpr int kRowsSeries = 3;    // the series form starts at the first level of at most 3 N frames, N the class's events
+constexpr int kRowsSeries = 3;    // the series form starts at the first level of at most 3 N frames (level 0: half that), N the class's events
 static_assert(kRowSlack >= 64 * 16, "a row kernel reads up to its capacity past a row's first event");
 
 // One length class: its rows and how a wave lays them out.
@@ -187,11 +192,11 @@ __device__ __forceinline__ uint32_t dot2(uint32_t a, uint32_t b, uint32_t c)
 }
 
 // Lag sums of one level's series (x: nw words of two 16-bit values between
-// kSeriesPad words of zeros, 16-byte aligned) for lags DPL + 1 .. 2 DPL.  The
+// kSeriesPad words of zeros, 16-byte aligned) for lags LO .. LO + DPL - 1.  The
 // group's lanes take consecutive stretches of whole 8-word blocks (two 16-byte
 // reads each) with the 8 words before a stretch in registers (win: words, sh:
 // the same one frame earlier); the group's last lane stores the sums.
-template <int G, int DPL>
+template <int G, int DPL, int LO>
 __device__ __forceinline__ void series_lags(const uint32_t* x, int nw, int h, uint32_t* out)
 {
     constexpr int U = 8;
@@ -219,13 +224,15 @@ __device__ __forceinline__ void series_lags(const uint32_t* x, int nw, int h, ui
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const uint32_t prev = u > 0 ? cur[u > 0 ? u - 1 : 0] : win[U - 1];
+                const uint32_t here = __builtin_amdgcn_alignbit(cur[u], prev, 16);
+                if constexpr (LO == 1) sh[u] = here;   // lag 1's
 #pragma unroll
                 for (int l = 0; l < DPL; l++) {
-                    const int lag = DPL + 1 + l;
+                    const int lag = LO + l;
                     const int m = lag / 2;   // even lag 2 m: word k - m; odd lag 2 m + 1: sh of word k - m
                     acc[l] = dot2(cur[u], (lag & 1) ? sh[(u + U - m) % U] : win[(u + U - m) % U], acc[l]);
                 }
-                sh[u] = __builtin_amdgcn_alignbit(cur[u], prev, 16);
+                sh[u] = here;
                 win[u] = cur[u];
             }
         }
@@ -282,7 +289,7 @@ constexpr int kWidePad = 16;
 // series_lags for a wide row: a word per value (x: nw words between kWidePad
 // words of zeros).  Values are at most 1024 x 65535, so products and sums
 // (at most total^2) are whole numbers below 2^53, exact in FP64.
-template <int G, int DPL>
+template <int G, int DPL, int LO>
 __device__ __forceinline__ void wide_series_lags(const uint32_t* x, int nw, int h, unsigned long long* out)
 {
     constexpr int U = 8, W = 2 * DPL;
@@ -308,7 +315,7 @@ __device__ __forceinline__ void wide_series_lags(const uint32_t* x, int nw, int 
             for (int u = 0; u < U; u++)
 #pragma unroll
                 for (int l = 0; l < DPL; l++) {
-                    const int lag = DPL + 1 + l;
+                    const int lag = LO + l;
                     acc[l] = fma(cur[u], u >= lag ? cur[u >= lag ? u - lag : 0] : win[u >= lag ? 0 : W + u - lag], acc[l]);
                 }
 #pragma unroll
@@ -340,19 +347,25 @@ __device__ __forceinline__ void wide_series_bin(uint32_t* x, int nx, int h)
 }
 
 // A wave's rows: lane group g has row p (-1: none), n events from `base` on.
-// A0, B0: the wave's LDS.  Narrow form: returns the mask of the wave's rows
-// that are wide (bit g), whose sums it leaves.  Wide form: counts of 16 bits
-// and any total, boundary slots and series of 32, lag sums of 64 bits.
-template <int G, int E, int DPL, bool WIDE>
-__device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& k, uint32_t* A0, uint32_t* B0, int32_t p,
-                                            int64_t base, int n)
+// A0, B0: the wave's LDS.  Narrow forms: store the mask of the wave's rows that
+// are wide (bit g), if any, to *flag and leave their sums; one for the series from a level
+// above 0 on, one for all levels (together in one kernel they cost it 1 to 2 %
+// in spilled scalar registers).  Wide form: counts of 16 bits and any total,
+// boundary slots and series of 32, lag sums of 64 bits.
+enum RowsForm { kRowsNarrow, kRowsNarrowSeries, kRowsWide };
+
+template <int G, int E, int DPL, RowsForm FORM>
+__device__ __forceinline__ void mt_rows(const RowsArgs& a, const RowsClass& k, uint32_t* A0, uint32_t* B0, int32_t p,
+                                        int64_t base, int n, uint8_t* flag)
 {
+    constexpr bool WIDE = FORM == kRowsWide;
     constexpr int R = kWave / G;
     constexpr int N = E * G;
     using Acc = std::conditional_t<WIDE, unsigned long long, uint32_t>;
     const int lane = lane_id();
     const int g = lane / G, h = lane % G;
-    const int T = a.T, aw = k.aw, bw = k.bw, ldeep = k.ldeep;
+    const int T = a.T, aw = k.aw, bw = k.bw;
+    const int ldeep = FORM == kRowsNarrowSeries ? 0 : k.ldeep;
     uint32_t* A = A0 + g * aw;
     uint32_t* B = B0 + g * bw;
     const int nbw = WIDE ? a.nb + 1 : a.nb / 2 + 1;   // words of the boundary slots 0 .. nb
@@ -378,7 +391,6 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
     }
     tot = group_sum<G>(tot);
     bool leave;            // another kernel's row
-    uint32_t wide_mask = 0u;
     if constexpr (WIDE) {
         const uint64_t bm = __ballot(big);
         leave = ((bm >> (g * G)) & (~0ull >> (64 - G))) != 0ull;
@@ -395,16 +407,18 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
         leave = tot > 65535u;
         const uint64_t wm = __ballot(leave && p >= 0);
         if (wm != 0ull) {
+            uint32_t wide_mask = 0u;
             // the next launch reads it: a store that stays in the L2 (one at
             // device scope went to memory, 30 ns each, 4 ms on a million rows)
             if (lane == 0) __hip_atomic_store(a.any_wide, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #pragma unroll
             for (int r = 0; r < R; r++) wide_mask |= (uint32_t)((wm >> (r * G)) & 1ull) << r;
+            if (lane == 0) *flag = (uint8_t)wide_mask;
         }
     }
     if (leave) p = -1;
     const uint64_t ok = __ballot(p >= 0);
-    if (ok == 0ull) return wide_mask;
+    if (ok == 0ull) return;
     wave_sync();
 #pragma unroll
     for (int i = 0; i < E; i++) B[slot_of<E>(i * G + h)] = leave ? kPad : e[i];
@@ -473,7 +487,7 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
                 const uint32_t ip = m[kPer * rr * aw + b.x];
                 const uint32_t jf = (uint32_t)m[kPer * rr * aw + b.z] - (uint32_t)m[kPer * rr * aw + b.y];
                 if ((ok >> (rr * G)) & 1ull) {
-                    const int64_t row0 = (int64_t)__builtin_amdgcn_readlane(p, rr * G) * T;
+                    const uint64_t row0 = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(p, rr * G) * (uint32_t)T;
                     if (a.w32) {
                         (reinterpret_cast<uint32_t*>(a.IP) + row0)[t] = ip;
                         (reinterpret_cast<uint32_t*>(a.IF) + row0)[t] = jf;
@@ -491,7 +505,7 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
     // ---- event pairs of the levels below ldeep: the lanes step over the
     // wave's events, a lane's row changing with every step, so that rows
     // with many pairs spread over the wave
-    if (ldeep > 0) {
+    if (FORM == kRowsNarrow || ldeep > 0) {
         const uint32_t dlim = (uint32_t)(2 * DPL + 1) << (ldeep - 1);
         const uint32_t fc = ((uint32_t)a.F >> (ldeep - 1)) << (ldeep - 1);   // whole frames of every level
         // events to visit: the longest row's, in steps of G
@@ -552,8 +566,12 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
         wave_sync();
         for (int L = ldeep; L < a.nlev; L++) {
             Acc* out = reinterpret_cast<Acc*>(A) + (L + 1) * DPL;
-            if constexpr (WIDE) wide_series_lags<G, DPL>(X, lf, h, out);
-            else series_lags<G, DPL>(X, (lf + 1) / 2, h, out);
+            if (FORM != kRowsNarrow && L == 0) {   // lags 1 .. dpl as well
+                if constexpr (WIDE) wide_series_lags<G, DPL, 1>(X, lf, h, out - DPL);
+                else series_lags<G, DPL, 1>(X, (lf + 1) / 2, h, out - DPL);
+            }
+            if constexpr (WIDE) wide_series_lags<G, DPL, DPL + 1>(X, lf, h, out);
+            else series_lags<G, DPL, DPL + 1>(X, (lf + 1) / 2, h, out);
             lf >>= 1;
             wave_sync();
             if (L + 1 < a.nlev) {
@@ -571,14 +589,13 @@ __device__ __forceinline__ uint32_t mt_rows(const RowsArgs& a, const RowsClass& 
             for (int rr = 0; rr < R; rr++) {
                 const uint64_t v = reinterpret_cast<const Acc*>(A0 + rr * aw)[t];
                 if ((ok >> (rr * G)) & 1ull) {
-                    const int64_t row0 = (int64_t)__builtin_amdgcn_readlane(p, rr * G) * T;
+                    const uint64_t row0 = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(p, rr * G) * (uint32_t)T;
                     (a.G2 + row0)[t] = (int64_t)v;
                 }
             }
         }
     }
     wave_sync();
-    return wide_mask;
 }
 
 // Row r of a class, for the lane's group: its pixel, first event and length (n
@@ -599,7 +616,7 @@ __device__ __forceinline__ void class_row(const RowsArgs& a, const RowsClass& k,
     else n = (int)len;
 }
 
-template <int G, int E, int DPL>
+template <int G, int E, int DPL, RowsForm FORM>
 __global__ void __launch_bounds__(kWave * kRowsWaves)
 k_mt_rows(const RowsArgs a, const RowsClass k)
 {
@@ -617,9 +634,8 @@ k_mt_rows(const RowsArgs a, const RowsClass k)
         int64_t base;
         int n;
         class_row<E * G>(a, k, r, r < nrows, p, base, n);
-        uint32_t wide = 0u;
-        if (__ballot(p >= 0) != 0ull) wide = mt_rows<G, E, DPL, false>(a, k, A0, B0, p, base, n);
-        if (lane == 0) k.wide[r0 / R] = (uint8_t)wide;
+        uint8_t* const flag = k.wide + r0 / R;
+        if (__ballot(p >= 0) != 0ull) mt_rows<G, E, DPL, FORM>(a, k, A0, B0, p, base, n, flag);
     }
 }
 
@@ -632,8 +648,8 @@ k_mt_rows(const RowsArgs a, const RowsClass k)
 // 143 registers allow three waves per SIMD.  Measured on jobs whose rows are
 // all wide, the whole pass, against a wave per row (the register and LDS
 // kernels of k_multitau.hip): 1024 x 1024 x 10,000 frames, 50 events a row,
-// dpl 8: 2.56 -> 2.38 ms (this kernel 1.2); 600 x 600 x 12,000, 293 a row,
-// dpl 4: 5.7 -> 3.4 ms; 512 x 384 x 6000, 690 a row: 9.8 -> 6.9 ms; 256 x 256 x
+// dpl 8: 2.56 -> 2.36 ms (this kernel 1.2); 600 x 600 x 12,000, 293 a row,
+// dpl 4: 5.7 -> 3.4 ms; 512 x 384 x 6000, 690 a row: 9.8 -> 7.2 ms; 256 x 256 x
 // 1000, 91 a row: 0.47 -> 0.39 ms.  (Listed one by one, with an atomic each, for
 // k_mt_sparse<1024>, these rows took 18.7, 14.3, 20.4 and 1.4 ms.)
 constexpr int kWideFlags = 8;
@@ -679,7 +695,7 @@ __device__ __forceinline__ void wide_class(const RowsArgs& a, const RowsClass& k
             int64_t base;
             int n;
             class_row<E * G>(a, k, (f0 + (b >> 3)) * R + (b & 7), in, p, base, n);
-            if (__ballot(p >= 0) != 0ull) mt_rows<G, E, DPL, true>(a, k, A0, B0, p, base, n);
+            if (__ballot(p >= 0) != 0ull) mt_rows<G, E, DPL, kRowsWide>(a, k, A0, B0, p, base, n, nullptr);
         }
         wave_sync();
     }
@@ -706,18 +722,21 @@ k_mt_rows_wide(const WideArgs a, int32_t lds_words)
 }  // namespace
 
 // First level of the series form for rows of at most N events: the first
-// level L >= 1 of at most 3 N binned frames, where a full row has an event in
+// level of at most 3 N binned frames, where a full row has an event in
 // every third frame and the series costs about what its event pairs do (2 N
 // and 6 N: 0.69 and 0.71 against 0.61 ms for the <= 64-event rows of the
 // 1 Mpx job, 1.46 and 1.64 against 1.42 ms for the 129..512-event rows of the
 // 600 x 600 x 12,000-frame job), or of at most deep_frames (tuning; negative:
-// none, the level count).
+// none, the level count).  Level 0 has twice the lags, so it begins there with
+// at most 3 N / 2 frames (with 3 N, rows of 129 events in 1536 frames would sum
+// a series of three times their pairs' work).
 int rows_series_level(const xpcs_mt_plan* p, int N)
 {
     const HostTables& h = p->h;
     const int nlev = (int)h.levels.size();
     if (p->tune.deep_frames < 0) return nlev;
     const int lim = p->tune.deep_frames > 0 ? p->tune.deep_frames : kRowsSeries * N;
+    if (h.levels[0].lf <= (p->tune.deep_frames > 0 ? lim : lim / 2)) return 0;
     for (int L = 1; L < nlev; L++)
         if (h.levels[(size_t)L].lf <= lim) return L;
     return nlev;
@@ -744,7 +763,8 @@ bool rows_supported(const xpcs_mt_plan* p)
                    : (lp.lo != h.dpl + 1 || lp.first != (L + 1) * h.dpl || lp.count > h.dpl))
             return false;
     }
-    const int64_t dlim = (int64_t)(2 * h.dpl + 1) << (rows_series_level(p, 16 * 4) - 1);
+    const int L = rows_series_level(p, kWave);
+    const int64_t dlim = L > 0 ? (int64_t)(2 * h.dpl + 1) << (L - 1) : 0;
     return (int64_t)h.F + dlim <= 65535;
 }
 
@@ -782,7 +802,7 @@ size_t rows_wide_flags(const xpcs_mt_plan* p)
 {
     size_t n = 0;
     for (int R : {8, 4, 2, 1}) n += wide_flag_bytes(p->h.P, R);
-    return n;
+    return (n + 15) / 16 * 16;
 }
 
 // Layout of the class of at most N events, G lanes to a row.
@@ -819,7 +839,8 @@ static void launch_rows_class(xpcs_mt_plan* p, hipStream_t s, int max_blocks)
     const size_t lds = sizeof(uint32_t) * (size_t)(kRowsWaves * R * (k.aw + k.bw));
     const int64_t need = ((int64_t)p->h.P + R * kRowsWaves - 1) / (R * kRowsWaves);
     const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(need, max_blocks));
-    k_mt_rows<G, E, DPL><<<nb, kWave * kRowsWaves, lds, s>>>(rows_args(p), k);
+    if (k.ldeep == 0) k_mt_rows<G, E, DPL, kRowsNarrowSeries><<<nb, kWave * kRowsWaves, lds, s>>>(rows_args(p), k);
+    else k_mt_rows<G, E, DPL, kRowsNarrow><<<nb, kWave * kRowsWaves, lds, s>>>(rows_args(p), k);
 }
 
 template <int DPL>
@@ -835,9 +856,9 @@ static void launch_rows_wide(xpcs_mt_plan* p, hipStream_t s)
     }
     const int64_t need = ((int64_t)p->h.P + 8 * kRowsWaves - 1) / (8 * kRowsWaves);
     const size_t lds = sizeof(uint32_t) * (size_t)(kRowsWaves * words);
-    // four rounds of what the chip holds at once (six workgroups a CU by registers): whole waves of long rows
-    // balance better than in one (690 events a row: 6.9 against 7.2 ms), and an empty launch takes no longer
-    const int64_t fit = 4 * 256 * std::min<int64_t>(6, (int64_t)((160 << 10) / lds));
+    // what the chip holds at once (six workgroups a CU by registers); four such rounds balance whole waves of
+    // long rows better (690 events a row: 6.9 against 7.2 ms), but cost every job without wide rows 4 us
+    const int64_t fit = 256 * std::min<int64_t>(6, (int64_t)((160 << 10) / lds));
     const unsigned nb = (unsigned)std::max<int64_t>(1, std::min(need, fit));
     k_mt_rows_wide<DPL><<<nb, kWave * kRowsWaves, lds, s>>>(w, words);
 }
