@@ -44,6 +44,30 @@ def test_rows_then_fewer_imm_events(xmt, orc, first):
     plan.close()
 
 
+def test_refused_frames_leave_the_data(xmt, orc):
+    """Frames refused for a value leave the plan's data as it was, also where
+    they would have needed a larger buffer."""
+    c = cases.sparse_case(mu=0.05, seed=21)
+    plan = xmt.Plan(c["W"], c["H"], c["F"], c["dpl"], c["dq"], c["sq"])
+    frames = np.ones((c["F"], c["W"] * c["H"]), np.uint32)
+    frames[-1, -1] = 65536
+    with pytest.raises(xmt.XpcsError, match="UNSUPPORTED"):
+        plan.ingest_frames(frames)
+    with pytest.raises(xmt.XpcsError, match="STATE"):
+        plan.execute()
+    plan.ingest_imm(c["imm"])
+    with pytest.raises(xmt.XpcsError, match="UNSUPPORTED"):
+        plan.ingest_frames(frames)
+    plan.execute()
+    check(plan, orc.run_exact(c["imm"], c["dq"], c["sq"], c["F"], c["dpl"]))
+    frames[-1, -1] = 65535
+    plan.ingest_frames(frames)
+    plan.execute()
+    want = frames.astype(np.uint16)
+    check(plan, orc.run_exact(synth.imm_bytes_dense(want, c["W"], c["H"]), c["dq"], c["sq"], c["F"], c["dpl"]))
+    plan.close()
+
+
 def busy_stream():
     """A torch stream with a tenth of a second of work queued."""
     import torch

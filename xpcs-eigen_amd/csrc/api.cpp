@@ -759,6 +759,7 @@ extern "C" xpcs_status xpcs_mt_ingest_imm(xpcs_mt_plan* p, const void* imm, size
     const size_t len = hi - lo;
     // the tail pad keeps tile loads of the last frame inside the allocation
     const size_t pad = 256;
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
     st = reserve(&p->d_imm_owned, &p->imm_cap, len + pad);
     if (st) return st;
     st = h2d_staged(p, p->d_imm_owned, b + lo, len);
@@ -832,6 +833,7 @@ extern "C" xpcs_status xpcs_mt_ingest_events(xpcs_mt_plan* p, const int32_t* pix
         }
     }
     const size_t pad = 256;
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
     st = reserve(&p->d_imm_owned, &p->imm_cap, bytes + pad);
     if (st) return st;
     st = h2d_staged(p, p->d_imm_owned, buf.data(), bytes);
@@ -890,6 +892,7 @@ extern "C" xpcs_status xpcs_mt_ingest_imm_device(xpcs_mt_plan* p, const void* de
     }
     p->clock.clear();
     p->ticks.clear();
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
     p->d_imm = static_cast<const uint8_t*>(dev_imm);
     std::vector<int64_t> so(sel.size());
     std::vector<uint32_t> sd(sel.size());
@@ -934,6 +937,7 @@ extern "C" xpcs_status xpcs_mt_ingest_packed(xpcs_mt_plan* p, const void* words,
         }
     }
     const size_t len = (size_t)(hi - lo) * (size_t)wb;
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
     st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
     if (st) return st;
     st = h2d_staged(p, p->d_imm_owned, static_cast<const uint8_t*>(words) + (size_t)lo * (size_t)wb, len);
@@ -983,22 +987,23 @@ extern "C" xpcs_status xpcs_mt_ingest_frames(xpcs_mt_plan* p, const void* frames
     const int64_t npd = (int64_t)h.W * h.H;
     const int64_t f_lo = sel.front(), f_hi = sel.back() + 1;
     const size_t len = (size_t)(f_hi - f_lo) * (size_t)npd * 2;
-    st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
-    if (st) return st;
-    if (bytes_per_value == 2) {
-        st = h2d_staged(p, p->d_imm_owned, static_cast<const uint8_t*>(frames) + (size_t)f_lo * npd * 2, len);
-    } else {
+    const uint8_t* values = static_cast<const uint8_t*>(frames) + (size_t)f_lo * npd * 2;
+    std::vector<uint16_t> nar;
+    if (bytes_per_value == 4) {
         // 32-bit values narrowed on the host (the kernels read 16-bit values)
         const uint32_t* src = static_cast<const uint32_t*>(frames) + (size_t)f_lo * npd;
-        std::vector<uint16_t> nar((size_t)(f_hi - f_lo) * (size_t)npd);
+        nar.resize((size_t)(f_hi - f_lo) * (size_t)npd);
         for (size_t i = 0; i < nar.size(); i++) {
             if (src[i] > 65535u)
                 return fail(XPCS_ERR_UNSUPPORTED, "ingest_frames: value %u at frame %lld exceeds 65535", src[i],
                             (long long)(f_lo + (int64_t)(i / (size_t)npd)));
             nar[i] = (uint16_t)src[i];
         }
-        st = h2d_staged(p, p->d_imm_owned, reinterpret_cast<const uint8_t*>(nar.data()), len);
+        values = reinterpret_cast<const uint8_t*>(nar.data());
     }
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
+    st = reserve(&p->d_imm_owned, &p->imm_cap, len + 256);
+    if (!st) st = h2d_staged(p, p->d_imm_owned, values, len);
     if (st) return st;
     p->d_imm = p->d_imm_owned;
     st = dense_prepare(p, nullptr, {});
@@ -1066,6 +1071,7 @@ extern "C" xpcs_status xpcs_mt_ingest_rows(xpcs_mt_plan* p, const int64_t* row_o
         if (row_off[j + 1] - row_off[j] <= reg_cap() && tot > 0xFFFFFFFFull) wide = true;
         if (row_off[j + 1] - row_off[j] <= kSparseCap && most > 65535u) big_rows++;
     }
+    p->mode = 0;   // the previous data goes: on failure nothing is ingested
     const xpcs_status st = reserve(&p->d_ev, &p->ev_cap, ev.size() + kRowSlack);
     if (st) return st;
     if (!ev.empty())
